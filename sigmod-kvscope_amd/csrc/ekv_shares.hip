@@ -23,14 +23,15 @@
 // thread sums (or maxes) its block's shares over its layers and query rows in a fixed order, and
 // the group partials are combined in LDS in a fixed order.
 //
-// Three forms.  Without a workspace one 1024-thread workgroup takes a whole row, so the longest row
-// sets the time (its records are read twice by one CU).  With a workspace (ekv_tile_shares_ws)
-// the layers are split into K groups whose workgroups write per-block partial sums (or maxes) and
-// their contributor counts: for 4 query rows and rows of at most 512 blocks (shares_wave_kernel)
-// the last of a row's workgroups to finish adds them and writes the row, otherwise a second kernel
-// (combine_kernel) adds each row's K partials in group order.  Every form adds in a fixed order,
-// so the results are the same on every call (the wave form's arrival counter only picks which
-// workgroup adds the partials).
+// Four forms.  Without a workspace one 1024-thread workgroup takes a whole row, so the longest row
+// sets the time (its records are read twice by one CU).  With a workspace (ekv_tile_shares_ws): for 4
+// query rows and rows of at most 512 blocks (shares_wave_kernel) the layers are split into groups and
+// the last of a row's workgroups to finish adds their per-block partials and writes the row; otherwise
+// the records stream through two kernels (stats_kernel, apply_kernel); where that form does not apply
+// or is the slower one, layer groups write per-block partials and their contributor counts and a second
+// kernel (combine_kernel) adds each row's K partials in group order.  Every form adds in a fixed
+// order, so the results are the same on every call (the arrival counters only pick which workgroup
+// finishes a row).
 #include <limits.h>
 #include <math.h>
 
@@ -76,6 +77,13 @@ struct Params {
   int32_t *status;     // wave form: the workspace's sticky status word (non-zero after a lost slot)
   int32_t spin_limit;  // wave form: reloads of a slot before its value is taken as lost
   int32_t lose;        // wave form, for tests of the failure path: no slot is ever seen as landed
+  int32_t nrows;
+  int32_t period;       // stream form: units of a block
+  int32_t slices;       // stream form: slices of a record (stats_kernel)
+  int32_t slice_units;  // stream form: units of a slice
+  int32_t chunks;       // stream form: workgroups of a row (apply_kernel)
+  int32_t columns;      // stream form: columns of units in a workgroup (apply_kernel)
+  struct Stat *stats;   // stream form: [rows][layers][slices][cells]
 };
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -103,6 +111,11 @@ struct RowWeight {
     return carries ? (b >= tail_start ? lw * tail_mult : lw) : 0.0f;
   }
 };
+
+// whether a record carries weight (RowWeight's rule on planes of m and l): m finite, l positive and finite
+__device__ __forceinline__ bool carries(float m, float l) {
+  return __builtin_amdgcn_classf(m, 0x1F8) && __builtin_amdgcn_classf(l, 0x180);
+}
 
 // merge two (max, sum w exp(m - max)) pairs
 __device__ __forceinline__ void merge(float &m, float &s, float m2, float s2) {
@@ -818,6 +831,472 @@ void shares_wave_kernel(const Params p) {
   }
 }
 
+// The stream form, for records the wave form does not take: two kernels that each stream the records
+// once, so that no per-layer partials are written.  stats_kernel reduces every (layer, query row) to
+// its peak and total; apply_kernel reads the records again (from the Infinity Cache when they fit
+// its 256 MB) and adds each block's shares over its layers and query rows in registers.  Both are bound
+// by the records' bandwidth once they are large (16 rows of U[256, 8192] blocks x 32 layers x 4 query
+// rows, 62 MB: ~17 us a kernel, 3.7 TB/s; a workgroup's chain of length, records and reduction is ~6 us)
+// and by that chain when small (~5 us a kernel).  The partial-sum kernels it replaces there, whose
+// combine runs on one workgroup a row, took 72 + 77 us.
+//
+// Records are read in units: 16-byte quads where the layout allows (V = 4: four query rows of a block
+// when the cells are a multiple of 4, four blocks when a block has one cell), else single floats
+// (V = 1).  C is the cells of a unit (4, or 1) and P = p.period the units of a block (1 for C = 1
+// quads).  A wave takes A = 64 / P * P units at a time, one per lane, so that a lane stays with its
+// C cells whatever the unit.
+constexpr int kStreamThreads = 256;  // stats_kernel: four waves
+constexpr int kApplyThreads = 512;   // apply_kernel: 8 waves, spread over layer groups and unit columns
+constexpr int kApplyWaves = kApplyThreads / kWave;
+constexpr int kMaxStreamStats = 2900;  // layers * cells: 46 KB of statistics in apply_kernel's LDS
+constexpr int kMaxRowStats = 16384;    // layers * cells * slices
+
+// exp(x) for x <= 0 (or -inf), 0 below e^-200.  exp2 of the rounded product x log2(e) alone is off by up
+// to |x| 2^-24; the product's remainder and log2(e)'s own are put back to first order.
+__device__ __forceinline__ float exp_near(float x) {
+  constexpr float kLog2e = 1.44269502f, kLog2eRest = 1.92596299e-8f, kLn2 = 0.693147181f;
+  x = x > -200.0f ? x : -200.0f;
+  const float y = x * kLog2e;
+  const float rest = fmaf(x, kLog2eRest, fmaf(x, kLog2e, -y));
+  const float v = __builtin_amdgcn_exp2f(y);
+  return fmaf(v, rest * kLn2, v);
+}
+
+// merge two (max, sum w exp(m - max)) pairs
+__device__ __forceinline__ void merge_near(float &m, double &s, float m2, double s2) {
+  const float M = fmaxf(m, m2);
+  if (M == -INFINITY) return;
+  s = s * exp_near(m - M) + s2 * exp_near(m2 - M);
+  m = M;
+}
+
+// wave_reduce4's sums in float64
+__device__ __forceinline__ double wave_sum4_f64(const float (&v)[4]) {
+  auto swap = [](uint32_t &x, uint32_t &y, auto rows16) {
+    asm volatile("" : "+v"(x), "+v"(y));
+    if constexpr (decltype(rows16)::value) {
+      const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+      x = r[0];
+      y = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+      x = r[0];
+      y = r[1];
+    }
+    asm volatile("" : "+v"(x), "+v"(y));
+  };
+  auto halves = [&](float a, float b) {  // lanes 0-31: a's two halves added, lanes 32-63: b's
+    uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+    swap(x, y, std::false_type{});
+    return (double)__builtin_bit_cast(float, x) + (double)__builtin_bit_cast(float, y);
+  };
+  auto words = [](double d, uint32_t &lo, uint32_t &hi) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, d);
+    lo = (uint32_t)b;
+    hi = (uint32_t)(b >> 32);
+  };
+  auto join = [](uint32_t lo, uint32_t hi) { return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo); };
+  uint32_t xl, xh, yl, yh;
+  words(halves(v[0], v[2]), xl, xh);
+  words(halves(v[1], v[3]), yl, yh);
+  swap(xl, yl, std::true_type{});
+  swap(xh, yh, std::true_type{});
+  double z = join(xl, xh) + join(yl, yh);
+  auto ror = [&](double d, auto ctrl) {
+    uint32_t lo, hi;
+    words(d, lo, hi);
+    return join((uint32_t)dpp_move<decltype(ctrl)::value>((int)lo), (uint32_t)dpp_move<decltype(ctrl)::value>((int)hi));
+  };
+  z += ror(z, std::integral_constant<int, 0x128>{});
+  z += ror(z, std::integral_constant<int, 0x124>{});
+  z += ror(z, std::integral_constant<int, 0x122>{});
+  z += ror(z, std::integral_constant<int, 0x121>{});
+  return z;
+}
+
+__device__ __forceinline__ double lane_value_f64(double d, int lane) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, d);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// A query row's peak and total over a slice.  One total divides every share of its query row, so a
+// lane's few terms are added in float32 but the lanes, waves and slices in float64, and it is stored as
+// two floats.
+struct Stat {
+  float peak, total, rest;
+};
+__device__ __forceinline__ Stat make_stat(float peak, double total) {
+  const float hi = (float)total;
+  return Stat{peak, hi, (float)(total - hi)};
+}
+
+// the units of a row of n blocks
+template <int V, int C>
+__device__ __forceinline__ int units_of(int n, int period) {
+  return V == 4 && C == 1 ? (n + 3) >> 2 : n * period;
+}
+
+template <int V>
+__device__ __forceinline__ void load_unit(const float *plane, int64_t base, int u, float (&x)[V]) {
+  if constexpr (V == 4) {
+    const f32x4_t q = *reinterpret_cast<const f32x4_t *>(plane + base + 4 * (int64_t)u);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = q[j];
+  } else {
+    x[0] = plane[base + u];
+  }
+}
+
+// The peak and total of every (layer, query row) over one slice of a row's units, by a workgroup (TEAM:
+// its four waves share the slice, waves taking A * K units in turn) or by one wave, into p.stats (peak
+// -inf: no weight in the slice).
+template <int V, int C, int K, bool TEAM>
+__global__ __launch_bounds__(kStreamThreads) void stats_kernel(const Params p) {
+  constexpr int kWaves = kStreamThreads / kWave;
+  constexpr int kUnitBlocks = V == 4 && C == 1 ? 4 : 1;  // blocks of a unit
+  __shared__ float s_m[TEAM ? kWaves : 1][kMaxCells];
+  __shared__ double s_t[TEAM ? kWaves : 1][kMaxCells];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const unsigned item = TEAM ? blockIdx.x : blockIdx.x * kWaves + wave;
+  const unsigned record = TEAM ? item / (unsigned)p.slices : item;
+  const int slice = TEAM ? (int)(item - record * (unsigned)p.slices) : 0;
+  const int out_row = (int)(record / (unsigned)p.layers), layer = (int)(record - (unsigned)out_row * p.layers);
+  if (!TEAM && out_row >= p.nrows) return;  // a wave past the last record (TEAM grids are exact)
+  const int src_row = p.row_ids != nullptr ? p.row_ids[out_row] : out_row;
+  const int n_row = p.row_blocks != nullptr ? max(p.row_blocks[out_row], 0) : p.width;
+  const int n = min(n_row, p.width);
+  const RowWeight weight(p, n_row);
+  const int P = p.period;
+  const int R = kWave / (unsigned)P, A = R * P;  // blocks (of P units) and units a wave takes at a time
+  const int row_in = lane / (unsigned)P;         // this lane's block among them
+  const bool active = lane < A;
+  const int units = units_of<V, C>(n, P);
+  const int first = slice * p.slice_units;
+  const int used = max(1u, (unsigned)(units + p.slice_units - 1) / (unsigned)p.slice_units);  // the row's slices with units
+  if (slice >= used) return;
+  const int end = min(units, first + p.slice_units);
+  const int64_t base = (int64_t)layer * p.layer_stride + (int64_t)src_row * p.row_stride;
+
+  float mx[C], sum[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    mx[c] = -INFINITY;
+    sum[c] = 0.0f;
+  }
+  for (int u0 = first + (TEAM ? wave * A * K : 0); u0 < end; u0 += (TEAM ? kWaves : 1) * A * K) {
+    float m[K][V], l[K][V];
+    // every load issued before any is used; a unit past the slice reads the row's first one
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int u = u0 + k * A + lane;
+      const int at = active && u < end ? u : 0;
+      load_unit<V>(p.m, base, at, m[k]);
+      load_unit<V>(p.l, base, at, l[k]);
+    }
+    // weights (0: the record carries none, its m then -inf), and the peaks
+    float top[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) top[c] = mx[c];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int u = u0 + k * A + lane;
+      const bool in = active && u < end;
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        const bool live = in && (C == 4 || V == 1 || 4 * u + j < n) && carries(m[k][j], l[k][j]);
+        m[k][j] = live ? m[k][j] : -INFINITY;
+        l[k][j] = live ? l[k][j] : 0.0f;
+        float &t = top[C == 4 ? j : 0];
+        t = m[k][j] > t ? m[k][j] : t;  // no NaN here: a plain compare
+      }
+    }
+    const int block_end = kUnitBlocks == 4 ? n : (unsigned)min(u0 + K * A, end) / (unsigned)P;
+    if (block_end > weight.tail_start) {  // the partial last tile's blocks (uniform: few waves hold any)
+      const int b0 = kUnitBlocks == 4 ? 0 : (int)((unsigned)u0 / (unsigned)P) + row_in;
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const int b = kUnitBlocks == 4 ? 4 * (u0 + k * A + lane) + j : b0 + k * R;
+          if (b >= weight.tail_start) l[k][j] *= weight.tail_mult;
+        }
+    }
+    // the totals against the new peaks (a cell with no weight yet: every term is 0 * exp(-inf) = 0)
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const float from = top[c] == -INFINITY ? 0.0f : top[c];
+      sum[c] *= exp_near(mx[c] - from);
+      mx[c] = top[c];
+      top[c] = from;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int j = 0; j < V; ++j) sum[C == 4 ? j : 0] += l[k][j] * exp_near(m[k][j] - top[C == 4 ? j : 0]);
+  }
+  // the lanes with the same cells reduced to lanes 0 .. P - 1 (rows 0 .. R - 1 of P lanes, halved)
+  float peak[C];
+  bool reduced = false;
+  if constexpr (C == 4) {
+    reduced = P == 1;
+    if (reduced) {
+      const float M = wave_reduce4<true>(mx);
+#pragma unroll
+      for (int c = 0; c < C; ++c) peak[c] = lane_value(M, 16 * c);
+    }
+  }
+  if (!reduced) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) peak[c] = mx[c];
+    for (int r = R; r > 1;) {
+      const int h = (r + 1) >> 1;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const float o = __shfl(peak[c], (lane + h * P) & (kWave - 1), kWave);
+        peak[c] = row_in < r - h ? fmaxf(peak[c], o) : peak[c];
+      }
+      r = h;
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) peak[c] = __shfl(peak[c], lane - row_in * P, kWave);
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) sum[c] = mx[c] == -INFINITY ? 0.0f : sum[c] * exp_near(mx[c] - peak[c]);
+  double total[C];
+  if constexpr (C == 4) {
+    if (reduced) {
+      const double t = wave_sum4_f64(sum);
+#pragma unroll
+      for (int c = 0; c < C; ++c) total[c] = lane_value_f64(t, 16 * c);
+    }
+  }
+  if (!reduced) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) total[c] = sum[c];
+    for (int r = R; r > 1;) {
+      const int h = (r + 1) >> 1;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const double o = __shfl(total[c], (lane + h * P) & (kWave - 1), kWave);
+        total[c] = row_in < r - h ? total[c] + o : total[c];
+      }
+      r = h;
+    }
+  }
+  Stat *stats = p.stats + (int64_t)item * p.cells;
+  if constexpr (!TEAM) {
+    if (lane < P)
+#pragma unroll
+      for (int c = 0; c < C; ++c) stats[lane * C + c] = make_stat(peak[c], total[c]);
+  } else {
+    if (lane < P)
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        s_m[wave][lane * C + c] = peak[c];
+        s_t[wave][lane * C + c] = total[c];
+      }
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c < p.cells) {
+      float M = -INFINITY;
+      double t = 0.0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) merge_near(M, t, s_m[w][c], s_t[w][c]);
+      stats[c] = make_stat(M, t);
+    }
+  }
+}
+
+// Each block's shares from the records and their peaks and totals: a workgroup takes `columns` columns
+// of A units of a row, 16 / columns waves a column, each over its layers (group g of LG:
+// [g layers / LG, (g + 1) layers / LG)); the groups' sums (or maxes) meet in LDS and are added in group
+// order.  The first records are requested before the statistics are read.  The row's last workgroup to
+// arrive clears the row's statistics, writes the blocks past the row and, for the max, renormalises
+// the row (written with device-coherent stores, complete before a workgroup counts its arrival).
+template <int V, int C>
+__global__ __launch_bounds__(kApplyThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void apply_kernel(const Params p) {
+  constexpr int kBlocksPer = V == 4 && C == 1 ? 4 : 1;  // blocks of a unit
+  constexpr int kDepth = V == 4 ? 4 : 8;                // layers in flight per lane
+  extern __shared__ float4 s_stat[];                    // [layers][cells]: peak, 1 / total in two parts
+  __shared__ double s_acc[kApplyThreads * kBlocksPer];  // [group][column][lane][block of the unit]
+  __shared__ double s_red[kApplyWaves];
+  __shared__ int s_count[kApplyWaves];
+  __shared__ int s_last;
+  const int out_row = (int)(blockIdx.x / (unsigned)p.chunks), chunk = (int)(blockIdx.x - out_row * (unsigned)p.chunks);
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int src_row = p.row_ids != nullptr ? p.row_ids[out_row] : out_row;
+  const int n_row = p.row_blocks != nullptr ? max(p.row_blocks[out_row], 0) : p.width;
+  const int n = min(n_row, p.width);
+  const RowWeight weight(p, n_row);
+  const bool use_max = p.aggregate == EKV_AGG_MAX;
+  const int P = p.period, cells = p.cells;
+  const int R = kWave / (unsigned)P, A = R * P;
+  const int columns = p.columns, LG = kApplyWaves / (unsigned)columns;
+  const int group = wave / (unsigned)columns, column = wave - group * columns;
+  const int units = units_of<V, C>(n, P);
+  const int u = (chunk * columns + column) * A + lane;  // this lane's unit
+  const bool in = lane < A && u < units;
+  const int b = kBlocksPer == 4 ? 4 * u : (int)((unsigned)u / (unsigned)P);  // its (first) block
+  const int cell0 = kBlocksPer == 4 ? 0 : (u - b * P) * C;
+  const int l0 = (unsigned)(group * p.layers) / (unsigned)LG, l1 = (unsigned)((group + 1) * p.layers) / (unsigned)LG;
+  const int64_t base = (int64_t)src_row * p.row_stride;
+  const int chunks = max(1, (units + columns * A - 1) / (columns * A));  // the row's chunks with units
+  if (chunk >= chunks) return;
+  const bool any = (chunk * columns + column) * A < units;  // the wave has a unit of the row
+
+  float m[kDepth][V], l[kDepth][V];
+  auto load = [&](int first) {  // layers first .. first + kDepth - 1 (past l1: layer l1 - 1 again)
+#pragma unroll
+    for (int k = 0; k < kDepth; ++k) {
+      const int64_t at = base + (int64_t)min(first + k, l1 - 1) * p.layer_stride;
+      load_unit<V>(p.m, at, in ? u : 0, m[k]);
+      load_unit<V>(p.l, at, in ? u : 0, l[k]);
+    }
+  };
+  const bool work = any && l0 < l1;
+  if (work) load(l0);
+
+  // the statistics (a query row's slices merged in order), and how many query rows carry any weight
+  int contributors = 0;
+  const int nstats = p.layers * cells;
+  const int slices = max(1u, (unsigned)(units + p.slice_units - 1) / (unsigned)p.slice_units);  // with units
+  Stat *stats = p.stats + (int64_t)out_row * p.slices * nstats;
+  for (int i = threadIdx.x; i < nstats; i += kApplyThreads) {
+    const int layer = (unsigned)i / (unsigned)cells;
+    const Stat *at = stats + (layer * p.slices * cells + (i - layer * cells));
+    float peak = at->peak;
+    double total = (double)at->total + at->rest;
+    for (int s0 = 1; s0 < slices; s0 += kBatch) {
+      Stat x[kBatch];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) x[k] = at[min(s0 + k, slices - 1) * cells];  // kBatch in flight
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k)
+        if (s0 + k < slices) merge_near(peak, total, x[k].peak, (double)x[k].total + x[k].rest);
+    }
+    const bool has = peak != -INFINITY;
+    const double inv = has ? 1.0 / total : 0.0;
+    s_stat[i] = make_float4(has ? peak : 0.0f, (float)inv, (float)(inv - (float)inv), 0.0f);
+    contributors += has ? 1 : 0;
+  }
+  contributors = wave_sum_int(contributors);
+  if (lane == 0) s_count[wave] = contributors;
+  __syncthreads();
+  // every thread has read the row's statistics: for the mean the workgroup counts its arrival here, and
+  // the answer is wanted only at the end
+  int arrived = 0;
+  auto arrive = [&] {
+    if (threadIdx.x == 0)
+      arrived = __hip_atomic_fetch_add(&p.arrivals[out_row], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (!use_max) arrive();
+  contributors = 0;
+#pragma unroll
+  for (int w = 0; w < kApplyWaves; ++w) contributors += s_count[w];
+
+  // The mean's sums: a few layers' shares in float32 pairwise, those sums in float64, so that the number
+  // of layers and query rows adds no error.
+  double acc[kBlocksPer];
+#pragma unroll
+  for (int j = 0; j < kBlocksPer; ++j) acc[j] = 0.0;
+  if (work) {
+    for (int first = l0; first < l1; first += kDepth) {
+      if (first > l0) load(first);
+      float part[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) part[j] = 0.0f;
+#pragma unroll
+      for (int k = 0; k < kDepth; ++k) {
+        if (first + k >= l1) break;
+        const float4 *st = s_stat + (first + k) * cells + cell0;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+          const float4 s = st[C == 4 ? j : 0];
+          // carries: its query row has a peak
+          const float w = carries(m[k][j], l[k][j]) ? l[k][j] * exp_near(m[k][j] - s.x) : 0.0f;
+          const float rest = w * s.z;
+          const float share = fmaf(w, s.y, rest);
+          part[j] = use_max ? (share > part[j] ? share : part[j]) : part[j] + share;
+        }
+      }
+      if constexpr (kBlocksPer == 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = use_max ? (part[j] > acc[j] ? part[j] : acc[j]) : acc[j] + part[j];
+      } else {
+        float p0 = part[0];
+        if constexpr (V == 4) {
+          const float top = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+          p0 = use_max ? top : (part[0] + part[1]) + (part[2] + part[3]);
+        }
+        acc[0] = use_max ? (p0 > acc[0] ? p0 : acc[0]) : acc[0] + p0;
+      }
+    }
+    // the partial last tile's blocks, and the blocks past the row
+#pragma unroll
+    for (int j = 0; j < kBlocksPer; ++j) {
+      const float tail = b + j >= weight.tail_start ? weight.tail_mult : 1.0f;
+      acc[j] = in && b + j < n ? acc[j] * tail : 0.0;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kBlocksPer; ++j) s_acc[threadIdx.x * kBlocksPer + j] = acc[j];
+  __syncthreads();
+
+  // block b of the chunk: its units' sums, over the layer groups in order
+  float *out = p.shares + (int64_t)out_row * p.shares_stride;
+  const int per_column = R * kBlocksPer;  // blocks of a column
+  const int chunk_blocks = columns * per_column;
+  for (int i = threadIdx.x; i < chunk_blocks; i += kApplyThreads) {
+    const int at = chunk * chunk_blocks + i;
+    if (at >= n) break;  // past the row: the last workgroup writes them
+    const int col = (unsigned)i / (unsigned)per_column, in_col = i - col * per_column;
+    double v = 0.0;
+    for (int g = 0; g < LG; ++g) {
+      const double *a = s_acc + (g * columns + col) * kWave * kBlocksPer + in_col * P;
+      for (int q = 0; q < P; ++q) v = use_max ? (a[q] > v ? a[q] : v) : v + a[q];
+    }
+    if (contributors == 0) v = NAN;  // no evidence about the row, tile_shares.py:103
+    else if (!use_max) v = v / contributors;
+    if (use_max) store_slot(reinterpret_cast<uint32_t *>(out + at), __builtin_bit_cast(uint32_t, (float)v));
+    else out[at] = (float)v;
+  }
+  if (use_max) {
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's stores have completed
+    __syncthreads();
+    arrive();
+  }
+  if (threadIdx.x == 0) s_last = arrived == chunks - 1;
+  __syncthreads();
+  if (!s_last) return;
+  if (threadIdx.x == 0) __hip_atomic_store(&p.arrivals[out_row], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int i = threadIdx.x; i < nstats * p.slices; i += kApplyThreads)  // every workgroup of the row has read them
+    stats[i] = Stat{0.0f, 0.0f, 0.0f};
+  for (int i = n + threadIdx.x; i < p.width; i += kApplyThreads) out[i] = contributors == 0 ? NAN : 0.0f;
+  if (use_max && contributors != 0) {  // renormalise the per-block max, tile_shares.py:97-100
+    double local = 0.0;
+    for (int i0 = threadIdx.x; i0 < n; i0 += kBatch * kApplyThreads) {
+      uint32_t x[kBatch];
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const int i = i0 + k * kApplyThreads;
+        x[k] = i < n ? load_slot(reinterpret_cast<const uint32_t *>(out + i)) : 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) local += __builtin_bit_cast(float, x[k]);
+    }
+    const double total = block_sum<kApplyThreads>(local, s_red);
+    for (int i = threadIdx.x; i < n; i += kApplyThreads) {
+      const float v = __builtin_bit_cast(float, load_slot(reinterpret_cast<const uint32_t *>(out + i)));
+      out[i] = total > 0.0 ? (float)(v / total) : 0.0f;
+    }
+  }
+}
+
 // The split form's second kernel: one workgroup per row combines the row's K partials in group
 // order, then applies the whole-row rules (NaN without evidence, the mean over contributing
 // pairs, or the max renormalised over the row).
@@ -893,6 +1372,70 @@ int g_lose = 0;
 // the register form's layers per group for J blocks per thread (at most 12 quads of each plane)
 constexpr int reg_layers(int J) { return J == 1 ? 8 : (J == 4 ? 2 : 4); }
 
+// The stream form where its statistics fit the workspace (3 floats a cell and slice in each
+// (row, layer)'s width of partials) and it is the faster one, else false with nothing launched.
+// Against the partial-sum forms, over 250 shapes of 1-256 rows, 16-8192 blocks, 1-48 layers, it is up to
+// 10 times as fast where it is taken (0.94-1 at the lines drawn here) and its error against float64 no
+// larger (2.4-6.6e-8, 4.5-14e-8 before).  Where it is not taken: 4 cells and at most 1024 blocks from 64
+// rows or 769 blocks on, whose records the register form reads once (below that 1.1-1.26 times; 0.93 at
+// 16 x 1024, 0.68-0.86 at 128 and 256 rows, whose combines fill the GPU); 4096 and more short records of
+// several cells (0.91-0.94 at 200 rows x 32 layers x 128 blocks x 8 cells); single floats below 2048
+// floats and 512 blocks a record (0.62-1.14, 1.1-7 from there on); records of one cell below 64 blocks
+// (0.9 at 3 x 16), for the max below 512 (0.92 at 240 x 232).
+bool launch_stream(Params p, int nrows, hipStream_t s) {
+  if (p.from_u || nrows > kMaxArrivalRows || (int64_t)p.layers * p.cells > kMaxStreamStats) return false;
+  const bool aligned = ((uintptr_t)p.m % 16) == 0 && ((uintptr_t)p.l % 16) == 0 && p.layer_stride % 4 == 0 &&
+                       p.row_stride % 4 == 0;
+  const bool quads = aligned && p.cells % 4 == 0;                        // four cells of a block
+  const bool blocks = aligned && p.cells == 1 && p.width % 4 == 0;       // four blocks of one cell
+  if (quads && p.cells == 4 && p.width <= 4 * kSplitThreads && (nrows >= 64 || p.width > 3 * kSplitThreads)) return false;
+  if (quads && (int64_t)nrows * p.layers >= 4096 && p.width * p.cells <= 2048) return false;
+  if (!quads && !blocks && p.width < 512 && p.width * p.cells < 2048) return false;
+  if (blocks && p.width < (p.aggregate == EKV_AGG_MAX ? 512 : 64)) return false;
+  p.nrows = nrows;
+  p.period = quads ? p.cells / 4 : blocks ? 1 : p.cells;
+  const int units = blocks ? p.width / 4 : p.width * p.period;
+  const int A = kWave / p.period * p.period;
+  const int64_t records = (int64_t)nrows * p.layers;
+  const int room = p.width / (3 * p.cells);  // slices whose statistics fit
+  if (room < 1) return false;
+  constexpr int kUnits = 4;  // units a lane has in flight
+  const bool team = units > A * kUnits;
+  const int most = (units + 4 * A * kUnits - 1) / (4 * A * kUnits);
+  // slices: enough workgroups to cover the GPU about eight times, while a row's statistics, which every
+  // workgroup of apply_kernel reads, stay within 192 KB
+  const int64_t want = (8 * (int64_t)cu_count() + records - 1) / records;
+  const int few = kMaxRowStats / (p.layers * p.cells);
+  p.slices = !team ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>({want, most, room, few}));
+  p.slice_units = ((units + p.slices - 1) / p.slices + 4 * A * kUnits - 1) / (4 * A * kUnits) * (4 * A * kUnits);
+  p.slices = (units + p.slice_units - 1) / p.slice_units;
+  p.stats = reinterpret_cast<Stat *>(p.part);
+  // apply_kernel: layer groups of waves until the workgroups cover the GPU about four times
+  auto chunks_of = [&](int columns) { return (units + columns * A - 1) / (columns * A); };
+  int groups = 1;
+  while (groups < kApplyWaves && 2 * groups <= p.layers &&
+         (int64_t)nrows * chunks_of(kApplyWaves / groups) < 4 * (int64_t)cu_count())
+    groups <<= 1;
+  p.columns = kApplyWaves / groups;
+  p.chunks = chunks_of(p.columns);
+  const int64_t grid1 = team ? records * p.slices : (records + 3) / 4, grid2 = (int64_t)nrows * p.chunks;
+  if (grid1 > INT_MAX || grid2 > INT_MAX) return false;
+  const size_t lds = (size_t)p.layers * p.cells * sizeof(float4);
+  auto run = [&](auto v_tag, auto c_tag) {
+    constexpr int V = decltype(v_tag)::value, C = decltype(c_tag)::value;
+    const dim3 g1((unsigned)grid1), t1(kStreamThreads);
+    if (team) hipLaunchKernelGGL((stats_kernel<V, C, kUnits, true>), g1, t1, 0, s, p);
+    else if (units <= A) hipLaunchKernelGGL((stats_kernel<V, C, 1, false>), g1, t1, 0, s, p);
+    else if (units <= 2 * A) hipLaunchKernelGGL((stats_kernel<V, C, 2, false>), g1, t1, 0, s, p);
+    else hipLaunchKernelGGL((stats_kernel<V, C, kUnits, false>), g1, t1, 0, s, p);
+    hipLaunchKernelGGL((apply_kernel<V, C>), dim3((unsigned)grid2), dim3(kApplyThreads), lds, s, p);
+  };
+  if (quads) run(std::integral_constant<int, 4>(), std::integral_constant<int, 4>());
+  else if (blocks) run(std::integral_constant<int, 4>(), std::integral_constant<int, 1>());
+  else run(std::integral_constant<int, 1>(), std::integral_constant<int, 1>());
+  return true;
+}
+
 // workspace null: one workgroup per row; otherwise the split form (workspace_bytes at least
 // split_workspace(nrows, width, layers))
 int launch(Params p, int nrows, void *workspace, size_t workspace_bytes, void *stream) {
@@ -958,6 +1501,7 @@ int launch(Params p, int nrows, void *workspace, size_t workspace_bytes, void *s
     else launch(std::integral_constant<int, 2 * kWaveLayers>());
     return check_hip(hipGetLastError(), "tile shares launch");
   }
+  if (split && launch_stream(p, nrows, s)) return check_hip(hipGetLastError(), "tile shares launch");
   if (split && vec && p.cells == 4 && p.width <= 4 * kSplitThreads) {
     // the register form: one pass, J blocks per thread, reg_layers(J) layers per group
     const int J = (p.width + kSplitThreads - 1) / kSplitThreads;

@@ -272,3 +272,38 @@ def test_a_lost_partial_sets_a_sticky_status_until_reset():
                 ekv_hip.call("ekv_tile_shares_reset", 0 if ws is None else ws.data_ptr(),
                              0 if ws is None else ws.numel(), 0)
                 ekv_hip.synchronize()
+
+
+@pytest.mark.parametrize("aggregate", ["mean", "max"])
+@pytest.mark.parametrize("layers,rows,width,cells", [
+    (3, 5, 2049, 4), (2, 3, 1028, 1), (5, 3, 2050, 1), (33, 2, 300, 8), (3, 4, 257, 7), (9, 3, 520, 7),
+    (2, 3, 200, 12), (4, 2, 130, 64), (40, 70, 700, 4), (1, 1, 8192, 4), (7, 2, 4096, 32), (1, 3, 4097, 2)])
+def test_records_streamed_in_units_match_the_oracle(layers, rows, width, cells, aggregate):
+    # the stream form: units of four query rows (1, 2, 3, 8 or 16 a block), of four blocks of one cell
+    # and of single floats; rows that end in a unit, a wave's units, a slice or a partial tile, empty
+    # rows, rows longer than the width, rows without evidence, unaligned rows.  Sums over at most
+    # 8192 blocks and 330 (layer, query row) pairs: within a few hundred float32 roundings of the mean
+    rng = np.random.default_rng(500 + layers + 3 * cells + width)
+    tile = 2
+    m = rng.normal(0, 3, (layers, rows, width, cells)).astype(np.float32)
+    l = rng.uniform(0.5, 30, (layers, rows, width, cells)).astype(np.float32)
+    l[rng.random(l.shape) < 0.02] = 0.0
+    l[rng.random(l.shape) < 0.01] = np.inf
+    m[rng.random(m.shape) < 0.03] = -np.inf
+    m[rng.random(m.shape) < 0.01] = np.nan
+    if layers > 1:
+        m[layers // 2, 0] = np.nan  # a layer without evidence
+    if rows > 2:
+        m[:, 1] = np.nan  # a row without evidence
+    lens = [width, width - 1, 1, 0, width + 3, 65, width // 2, 2 * (width // 4) + 1]
+    row_blocks = np.array([lens[i % len(lens)] for i in range(rows)])
+    planes = np.stack([m, l])
+    dev = planes_on_device(planes)
+    blocks = torch.from_numpy(row_blocks.astype(np.int32)).cuda()
+    workspace = torch.zeros(tile_shares.shares_workspace_bytes(rows, width, layers), dtype=torch.uint8, device="cuda")
+    got = [tile_shares.tile_shares(dev.data_ptr(), layers, layers, rows, width, cells, None, blocks, tile, aggregate,
+                                   workspace=workspace).cpu().numpy() for _ in range(2)]
+    assert np.array_equal(got[0], got[1], equal_nan=True)
+    assert int(torch.count_nonzero(workspace)) == 0
+    want = ots.normalize(ots.read_rows(planes, layers, np.arange(rows), tile), row_blocks, tile, aggregate)
+    assert_close(got[0].astype(np.float64), want, 1e-6, f"{layers} x {rows} x {width} x {cells}, {aggregate}")
