@@ -21,9 +21,9 @@
 //
 // maxmin: raise the lowest retained share as far as the budget allows, then spend what is left on
 // the lowest request first (observe/allocation.py:126-166).  Per request: the pinned shares' NumPy
-// sum (base), its open blocks in stable descending share order (a radix sort over the same
-// order-preserving keys, one workgroup per request, in LDS; past 12288 blocks in global memory), and
-// their running float64 totals, added in that order as np.cumsum does.  The 60-step bisection of the level: a request's count at a level is
+// sum (base), its open blocks in stable descending share order (by rank in buckets of the same
+// order-preserving keys, one workgroup per request, in LDS; a radix sort past 8192 blocks, in global
+// memory past 12288), and their running float64 totals, added in that order as np.cumsum does.  The 60-step bisection of the level: a request's count at a level is
 // min(1 + lower_bound(totals + 2 r, level - base - 1e-12 + 2 r), open), the shifted-by-2r comparison
 // NumPy's single search makes.  Its first 20 steps are walks over counts that two kernels sum over
 // every CU at the levels they can reach; the rest run in one workgroup, every request keeping the
@@ -33,6 +33,7 @@
 
 #include <limits.h>
 #include <math.h>
+#include <stddef.h>
 
 #include <algorithm>
 
@@ -71,6 +72,18 @@ struct RowStat {
   double total;  // NumPy's sum of the clamped scores
   int n, pinned, open, pad;
 };
+
+static_assert(sizeof(RowStat) == 24 && offsetof(RowStat, n) == 8 && offsetof(RowStat, open) == 16, "three words");
+
+// a request's statistics with device-coherent stores, for a later workgroup of the same launch
+__device__ __forceinline__ void store_row_stat(RowStat *at, const RowStat &st) {
+  unsigned long long *w = reinterpret_cast<unsigned long long *>(at);
+  const unsigned long long words[3] = {(unsigned long long)__double_as_longlong(st.total),
+                                       (unsigned long long)(uint32_t)st.n | ((unsigned long long)(uint32_t)st.pinned << 32),
+                                       (unsigned long long)(uint32_t)st.open};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) __hip_atomic_store(w + i, words[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 struct Params {
   const double *scores;
@@ -211,7 +224,8 @@ __global__ __launch_bounds__(kPrepThreads) void prepare_kernel(const Params p) {
 // the requests' pinned, existing and open blocks, summed over the rows' statistics by one
 // workgroup, then the budget's mode (allocation.py:57-76) and the select's start; the state
 // (histogram, flags, counters) is cleared first
-template <int NT>
+// COHERENT: the statistics were stored by this launch's other workgroups (store_row_stat).
+template <int NT, bool COHERENT = false>
 __device__ void decide(const Params &p) {
   __shared__ long long s_red[3][NT / kWave];
   {
@@ -220,7 +234,17 @@ __device__ void decide(const Params &p) {
   }
   long long v[3] = {0, 0, 0};  // must, sizes, open_total
   for (int r = threadIdx.x; r < p.rows; r += NT) {
-    const RowStat st = p.row_stat[r];
+    RowStat st;
+    if constexpr (COHERENT) {
+      unsigned long long *w = reinterpret_cast<unsigned long long *>(p.row_stat + r);
+      const unsigned long long a = __hip_atomic_load(w + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned long long b = __hip_atomic_load(w + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      st.n = (int)(uint32_t)a;
+      st.pinned = (int)(uint32_t)(a >> 32);
+      st.open = (int)(uint32_t)b;
+    } else {
+      st = p.row_stat[r];
+    }
     v[0] += st.pinned;
     v[1] += st.n;
     v[2] += st.open;
@@ -687,25 +711,25 @@ constexpr int kDigitBins = 256;
 constexpr int kIndexBits = 14;    // block indices below 2^14
 constexpr int kSortLowBits = 24;  // the key bits the first sort leaves out
 static_assert(kMaxWidth <= (1 << kIndexBits), "a block index fits the packed element");
-static_assert(kSortThreads == 4 * kDigitBins, "the count scan takes four counts of one digit a thread");
 
 template <int MAX_ITEMS>
 struct SortLds {
   unsigned long long elem[MAX_ITEMS * kSortThreads];
-  unsigned int count[kSortWaves][kDigitBins];  // per wave and digit; scratch between the passes
+  unsigned short count[kSortWaves][kDigitBins];  // per wave and digit; scratch between the passes
+  int resort;
 };
 
 // This wave's ranking of its ITEMS x 64 elements e (position order: i, then lane) by the digit at bit
 // lo: info[i] = digit (bits 16-23, descending as ascending) << 16 | the element's rank among the
 // wave's elements with that digit.  cnt (the wave's 256 counts in LDS) ends holding the wave's count
 // of each digit.  Every lane of the wave must take part.
-template <int ITEMS>
-__device__ __forceinline__ void rank_wave(const unsigned long long (&e)[ITEMS], int lo, unsigned int *cnt,
+template <int ITEMS, class COUNT>
+__device__ __forceinline__ void rank_wave(const unsigned long long (&e)[ITEMS], int lo, COUNT *cnt,
                                           uint32_t (&info)[ITEMS]) {
   const int lane = lane_id();
   // cleared before the counting below: one wave's LDS accesses take effect in order
 #pragma unroll
-  for (int j = 0; j < kDigitBins / kWave; ++j) cnt[j * kWave + lane] = 0u;
+  for (int j = 0; j < kDigitBins / kWave; ++j) cnt[j * kWave + lane] = (COUNT)0;
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const uint32_t d = 255u - (uint32_t)((e[i] >> lo) & 255u);
@@ -722,7 +746,7 @@ __device__ __forceinline__ void rank_wave(const unsigned long long (&e)[ITEMS], 
     // the wave's count of d so far, then every lane with d stores the same new count (no lane
     // diverges; this wave's LDS accesses take effect in order, so the next position reads it)
     const uint32_t before = cnt[d];
-    cnt[d] = before + (uint32_t)(__popc(peer_lo) + __popc(peer_hi));
+    cnt[d] = (COUNT)(before + (uint32_t)(__popc(peer_lo) + __popc(peer_hi)));
     info[i] = (d << 16) | (before + __builtin_amdgcn_mbcnt_hi(peer_hi, __builtin_amdgcn_mbcnt_lo(peer_lo, 0u)));
     // computed here: left to the compiler, the rank's parts (two masks and a count) would be carried
     // to the moves after the scan instead of this one word
@@ -730,9 +754,11 @@ __device__ __forceinline__ void rank_wave(const unsigned long long (&e)[ITEMS], 
   }
 }
 
-// One pass over bits [lo, lo + 8) of the ITEMS * kSortThreads elements in `elem`.
-template <int ITEMS>
-__device__ __forceinline__ void radix_pass(unsigned long long *elem, unsigned int (*count)[kDigitBins], int lo) {
+// One pass over bits [lo, lo + 8) of the ITEMS * NT elements in `elem`.
+template <int NT, int ITEMS>
+__device__ __forceinline__ void radix_pass(unsigned long long *elem, unsigned short (*count)[kDigitBins], int lo) {
+  static_assert(NT % kDigitBins == 0, "the count scan takes four counts of one digit a thread");
+  constexpr int kShare = NT / kDigitBins;  // threads of a digit
   const int lane = lane_id();
   const int wave = threadIdx.x / kWave;
   const int run0 = wave * kWave * ITEMS;
@@ -743,9 +769,9 @@ __device__ __forceinline__ void radix_pass(unsigned long long *elem, unsigned in
   rank_wave<ITEMS>(e, lo, count[wave], info);
   __syncthreads();  // every wave's counts are final and every element is in registers
   {
-    // the counts in (digit, wave) order: thread t takes digit t / 4 and waves 4 (t % 4) .. + 3; the
-    // scan's scratch is the element array, free until the elements move
-    const int d = threadIdx.x >> 2, w0 = (threadIdx.x & 3) * 4;
+    // the counts in (digit, wave) order: thread t takes digit t / kShare and waves 4 (t % kShare) .. + 3;
+    // the scan's scratch is the element array, free until the elements move
+    const int d = threadIdx.x / kShare, w0 = (threadIdx.x % kShare) * 4;
     uint32_t c[4];
     int sum = 0;
 #pragma unroll
@@ -754,10 +780,10 @@ __device__ __forceinline__ void radix_pass(unsigned long long *elem, unsigned in
       sum += (int)c[q];
     }
     int total;
-    int at = block_exclusive_scan<kSortThreads>(sum, reinterpret_cast<int *>(elem), total);
+    int at = block_exclusive_scan<NT>(sum, reinterpret_cast<int *>(elem), total);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      count[w0 + q][d] = (uint32_t)at;
+      count[w0 + q][d] = (unsigned short)at;
       at += (int)c[q];
     }
   }
@@ -775,20 +801,20 @@ __device__ __forceinline__ unsigned long long block_key(const RowStat &st, bool 
   return (b >= st.n || pinned) ? 0ull : k;
 }
 
-template <int ITEMS, int MAX_ITEMS>
-__device__ __forceinline__ void sort_request(const MaxminParams &m, const RowStat &st, int r, SortLds<MAX_ITEMS> &lds) {
-  static_assert(ITEMS <= MAX_ITEMS, "the LDS holds the sort");
+// The request's elements in sorted order in elem[0 .. NT * ITEMS), by NT threads.
+template <int NT, int ITEMS>
+__device__ __forceinline__ void radix_ranks(const MaxminParams &m, const RowStat &st, int r, unsigned long long *elem,
+                                            unsigned short (*count)[kDigitBins], int *resort) {
   constexpr unsigned long long kIndexMask = (1ull << kIndexBits) - 1ull;
   constexpr unsigned long long kLow = (1ull << kSortLowBits) - 1ull;
   const Params &p = m.p;
-  const int n = st.n, open = st.open;
+  const int n = st.n;
   const int tid = threadIdx.x;
   const double *srow = p.scores + (int64_t)r * p.scores_stride;
   // Every load is unconditional and in range (indices clamped to the request's last block; without an
   // explicit mask the pinned flags are read from the scores and ignored), so none waits in a branch.
   const bool masked = p.pinned != nullptr;
   const uint8_t *prow = masked ? p.pinned + (int64_t)r * p.pinned_stride : reinterpret_cast<const uint8_t *>(srow);
-  unsigned long long *elem = lds.elem;
   constexpr int kStep = ITEMS < 4 ? ITEMS : 4;  // positions loaded at a time
   // the full keys of the blocks that elements name, from their scores (in cache: just read), kStep
   // at a time with every load issued before any is used
@@ -813,20 +839,20 @@ __device__ __forceinline__ void sort_request(const MaxminParams &m, const RowSta
     uint8_t pin[kStep];
 #pragma unroll
     for (int i = 0; i < kStep; ++i) {  // every load issued before any is used
-      const int c = min((i0 + i) * kSortThreads + tid, n - 1);
+      const int c = min((i0 + i) * NT + tid, n - 1);
       score[i] = srow[c];
       pin[i] = prow[c];
     }
 #pragma unroll
     for (int i = 0; i < kStep; ++i) {
-      const int pos = (i0 + i) * kSortThreads + tid;
+      const int pos = (i0 + i) * NT + tid;
       const unsigned long long k = block_key(st, masked, pos, score[i], pin[i]);
       elem[pos] = ((k >> kSortLowBits) << kIndexBits) | (unsigned long long)pos;
     }
   }
   __syncthreads();
 #pragma unroll 1
-  for (int lo = kIndexBits; lo < kIndexBits + 64 - kSortLowBits; lo += 8) radix_pass<ITEMS>(elem, lds.count, lo);
+  for (int lo = kIndexBits; lo < kIndexBits + 64 - kSortLowBits; lo += 8) radix_pass<NT, ITEMS>(elem, count, lo);
 
   // Neighbours that tie in the top bits: each thread takes ITEMS consecutive positions (so that a
   // scan over the threads numbers the runs of equal top bits in order) and the full keys of their blocks.
@@ -839,11 +865,10 @@ __device__ __forceinline__ void sort_request(const MaxminParams &m, const RowSta
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) idx[i] = (int)(elem[t * ITEMS + i] & kIndexMask);
   keys_of(idx, key);
-  unsigned long long *last_key = reinterpret_cast<unsigned long long *>(&lds.count[0][0]);  // [kSortThreads]
-  unsigned int *resort = &lds.count[kSortWaves - 1][kDigitBins - 1];  // past last_key
-  static_assert(sizeof(unsigned long long) * kSortThreads < sizeof(lds.count), "the flag lies past last_key");
+  static_assert(sizeof(unsigned long long) * NT == sizeof(unsigned short) * NT / kWave * kDigitBins, "a key a thread");
+  unsigned long long *last_key = reinterpret_cast<unsigned long long *>(&count[0][0]);  // [NT]
   last_key[t] = key[ITEMS - 1];
-  if (t == 0) *resort = 0u;
+  if (t == 0) *resort = 0;
   __syncthreads();
   const unsigned long long before = t > 0 ? last_key[t - 1] : 0ull;
   {
@@ -854,10 +879,10 @@ __device__ __forceinline__ void sort_request(const MaxminParams &m, const RowSta
       const unsigned long long prev = i > 0 ? key[i - 1] : before;
       unsorted |= pos > 0 && pos < n && (key[i] >> kSortLowBits) == (prev >> kSortLowBits) && (key[i] & kLow) > (prev & kLow);
     }
-    if (unsorted) *resort = 1u;
+    if (unsorted) *resort = 1;
   }
   __syncthreads();
-  if (*resort != 0u) {
+  if (*resort != 0) {
     // each run of equal top bits again, on (bits 0-23, index): runs numbered in order by a scan of
     // their first positions, elements packed as (~run, bits 0-23, index) and sorted on bits 14-51
     // from the present order, which holds a run's blocks in block order
@@ -868,7 +893,7 @@ __device__ __forceinline__ void sort_request(const MaxminParams &m, const RowSta
       starts += (t * ITEMS + i == 0 || (key[i] >> kSortLowBits) != (prev >> kSortLowBits)) ? 1 : 0;
     }
     int total_runs;
-    int run = block_exclusive_scan<kSortThreads>(starts, reinterpret_cast<int *>(elem), total_runs) - 1;
+    int run = block_exclusive_scan<NT>(starts, reinterpret_cast<int *>(elem), total_runs) - 1;
 #pragma unroll
     for (int i = 0; i < ITEMS; ++i) {
       const unsigned long long prev = i > 0 ? key[i - 1] : before;
@@ -878,20 +903,30 @@ __device__ __forceinline__ void sort_request(const MaxminParams &m, const RowSta
     }
     __syncthreads();
 #pragma unroll 1
-    for (int lo = kIndexBits; lo < 2 * kIndexBits + kSortLowBits; lo += 8) radix_pass<ITEMS>(elem, lds.count, lo);
+    for (int lo = kIndexBits; lo < 2 * kIndexBits + kSortLowBits; lo += 8) radix_pass<NT, ITEMS>(elem, count, lo);
   }
+}
+
+template <int ITEMS, int MAX_ITEMS>
+__device__ __forceinline__ void sort_request(const MaxminParams &m, const RowStat &st, int r, SortLds<MAX_ITEMS> &lds) {
+  static_assert(ITEMS <= MAX_ITEMS, "the LDS holds the sort");
+  constexpr unsigned long long kIndexMask = (1ull << kIndexBits) - 1ull;
+  radix_ranks<kSortThreads, ITEMS>(m, st, r, lds.elem, lds.count, &lds.resort);
+  const Params &p = m.p;
+  const int n = st.n, open = st.open;
+  const double *srow = p.scores + (int64_t)r * p.scores_stride;
+  const bool masked = p.pinned != nullptr;
+  const uint8_t *prow = masked ? p.pinned + (int64_t)r * p.pinned_stride : reinterpret_cast<const uint8_t *>(srow);
   // the outputs, striped (coalesced stores): position i * kSortThreads + thread
   const int64_t row0 = (int64_t)r * p.width;
-  t = tid;
+  int t = threadIdx.x;
   asm volatile("" : "+v"(t));
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) idx[i] = (int)(elem[i * kSortThreads + t] & kIndexMask);
-  keys_of(idx, key);
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const int pos = i * kSortThreads + t;
-    if (pos < n) m.vals_out[row0 + pos] = idx[i];
-    if (pos < open) m.prefix[row0 + pos] = key_value(key[i]);
+    const int b = (int)(lds.elem[pos] & kIndexMask);
+    if (pos < n) m.vals_out[row0 + pos] = b;
+    if (pos < open) m.prefix[row0 + pos] = key_value(block_key(st, masked, b, srow[b], prow[b]));
   }
 }
 
@@ -912,7 +947,7 @@ __device__ void order_requests(const MaxminParams &m) {
   }
   if (tid < kOrderClasses) s_count[tid] = 0;
   __syncthreads();
-  auto cls = [&](int r) { return min(m.p.row_stat[r].n / kOrderStep, kOrderClasses - 1); };
+  auto cls = [&](int r) { return min(row_blocks(m.p, r) / kOrderStep, kOrderClasses - 1); };
   for (int r = tid; r < rows; r += kSortThreads) atomicAdd(&s_count[cls(r)], 1);
   __syncthreads();
   if (tid == 0) {
@@ -936,25 +971,19 @@ __global__ __launch_bounds__(kSortThreads) void mm_plan_kernel(const MaxminParam
   decide<kSortThreads>(m.p);
 }
 
-// Two 16-wave sorting workgroups share a CU where their LDS allows it (sorts of up to 8192 blocks take
-// 80 KB), at most 64 VGPRs each (8 waves per SIMD); the 12-key sort's 112 KB keeps it alone on a CU.
-template <int MAX_ITEMS>
-__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(MAX_ITEMS <= 8 ? 8 : 4)))
+// Rows of 8193 to kMaxWidth blocks (shorter ones: mm_rows_kernel): the 12-key sort's LDS keeps a
+// workgroup alone on a CU.
+__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void mm_sort_kernel(const MaxminParams m) {
-  __shared__ SortLds<MAX_ITEMS> lds;
+  constexpr int kItems = kMaxWidth / kSortThreads;
+  __shared__ SortLds<kItems> lds;
   const int r = m.order[blockIdx.x];
   const RowStat st = m.p.row_stat[r];
   if (st.n <= 0) return;
-  if (st.n <= kSortThreads)
-    sort_request<1>(m, st, r, lds);
-  else if (st.n <= 2 * kSortThreads)
-    sort_request<2>(m, st, r, lds);
-  else if (MAX_ITEMS == 4 || st.n <= 4 * kSortThreads)
-    sort_request<MAX_ITEMS < 4 ? MAX_ITEMS : 4>(m, st, r, lds);
-  else if (MAX_ITEMS == 8 || st.n <= 8 * kSortThreads)
-    sort_request<MAX_ITEMS < 8 ? MAX_ITEMS : 8>(m, st, r, lds);
-  else
-    sort_request<MAX_ITEMS>(m, st, r, lds);
+  if (st.n <= kSortThreads) sort_request<1>(m, st, r, lds);
+  else if (st.n <= 4 * kSortThreads) sort_request<4>(m, st, r, lds);
+  else if (st.n <= 8 * kSortThreads) sort_request<8>(m, st, r, lds);
+  else sort_request<kItems>(m, st, r, lds);
 }
 
 // Requests wider than a sort in LDS: the same radix sort, one workgroup per request, its elements in
@@ -1422,6 +1451,660 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
   __syncthreads();
   for (int j = threadIdx.x; j < kLevels; j += kTotalsThreads)
     if (s_count[j] > 0) atomicAdd(&m.level_count[j], s_count[j]);
+}
+
+// ---- a request in one workgroup --------------------------------------------------------------
+// For rows of at most 8192 blocks one workgroup takes a request from its scores to its level
+// positions, with its blocks in LDS and registers throughout: NumPy's total, the pinned shares' sum, the
+// sort, the running totals, and the positions of the levels j / kLevels in them.
+//
+// The sort places every open block by its exact rank, without passes over digits.  With x = (largest
+// key) - key, ascending in the sorted order, the blocks are counted in 511 coarse bins of x's leading
+// bits (zero and NaN shares in a bin of their own after them); a bin of c blocks is cut into about c / 2
+// to c / 4 buckets (two at least where the words below need it) of its next bits, so that a bucket holds a few blocks however the shares are spread;
+// and each block's rank is its bucket's first position plus the blocks of its bucket before it, counted
+// by comparing.  A bucket's bits fix all but x's low 51 bits (shares over more than 2^9 binades take the
+// radix sort), so those and the block's 13-bit index are one 64-bit word, and every comparison is of the
+// whole key and then the index: the order is the stable one whatever order the buckets were filled in.
+// Bucket bounds come from a bitmap of the buckets' first positions: a wave ranks 64 consecutive positions
+// and reads one word of it.  A request with a bucket of more than kBucketLimit blocks (many equal
+// shares, or shares that crowd together far below the bins' width) takes the radix sort instead.
+//
+// The running totals are scan_chunk's exact windows over the whole workgroup, in which only a new binade
+// ends a window (scan_window), so a long request takes ~5 windows.
+//
+// At 1024 x U[1, 8192]: 112 us, where the totals, the radix sort of every request and a scan wave and a
+// level wave a request took 12 + 99 + 55; at 128 x U[32, 512]: 17 us for 6 + 12 + 25.  Bound by a
+// request's chain of phases, each a few LDS round trips and dependent float64 operations between
+// barriers (~120000 cycles for 8192 blocks: loads 15, total 7, keys 7, ranks 45, totals 25, levels 7),
+// two 8-wave workgroups a CU (80 KB of LDS each) filling each other's gaps.  1024 threads a request at 64
+// VGPRs spilled (328 us); __syncthreads' waits for global stores cost ~5 us a request.
+constexpr int kRowsWidth = 8 * kSortThreads;  // the widest request
+static_assert(kRowsWidth <= 1 << 13, "a block index fits a bucket sort's word");
+constexpr int kCoarse = 512;                  // coarse bins; the last one holds the zero and NaN shares
+constexpr int kBucketLimit = 128;
+constexpr int kTies = 64;  // ties of a scan window resolved in place
+constexpr int kRowIndexBits = 13;             // block indices in a bucket sort's words
+
+template <int NT, int ITEMS>
+struct RowLds {
+  static constexpr int kCap = NT * ITEMS;
+  static constexpr int kBuckets = kCap / 2 + 2 * kCoarse;  // a bin of c blocks has at most max(2, c / 2)
+  union {
+    struct {
+      unsigned long long elem[kCap];
+      union {
+        unsigned int bucket[kBuckets / 2];             // two 16-bit counts, then first positions, a word
+        unsigned short count[NT / kWave][kDigitBins];  // the radix sort's
+      };
+    };
+    double share[kCap + kCap / 16];  // by chunk_slot; the pinned shares' list in order
+    unsigned short pos_of[kCap];
+  };
+  union {
+    PairwiseLds pair;
+    struct {
+      union {
+        unsigned int coarse[kCoarse];  // counts, then first bucket | bits << 16
+        double line[kWave];            // scan_row's values added one at a time
+      };
+      union {
+        unsigned long long scan64[NT / kWave][2];
+        double wave_sum[NT / kWave];
+        int scan[NT / kWave];
+      };
+    };
+  };
+  union {
+    uint32_t heads[kCap / 32 + 2];
+    int pin_count[NT / kWave * ITEMS];
+  };
+  double base;
+  int flag, stop, ties, tie[kTies];
+};
+
+// Keeps the compiler from interleaving one block's work with the next one's (eight blocks' at once spill).
+__device__ __forceinline__ void keep_order() { __builtin_amdgcn_sched_barrier(0); }
+
+// The thread index, opaque to the compiler: a phase that takes it this way has its addresses computed where
+// they are used (computed up front and held across the phases, they spill).
+__device__ __forceinline__ int phase_thread() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
+// The largest a and b over the workgroup, in every thread.
+template <int NT>
+__device__ __forceinline__ void block_max2_u64(unsigned long long &a, unsigned long long &b,
+                                               unsigned long long (*scratch)[2]) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    const unsigned long long x = __shfl_xor(a, m, kWave), y = __shfl_xor(b, m, kWave);
+    a = x > a ? x : a;
+    b = y > b ? y : b;
+  }
+  if (lane_id() == 0) {
+    scratch[threadIdx.x / kWave][0] = a;
+    scratch[threadIdx.x / kWave][1] = b;
+  }
+  lds_barrier();
+#pragma unroll
+  for (int w = 0; w < NT / kWave; ++w) {
+    a = scratch[w][0] > a ? scratch[w][0] : a;
+    b = scratch[w][1] > b ? scratch[w][1] : b;
+  }
+  lds_barrier();
+}
+
+// The exact ranks of a request's open blocks: pos_of[b] in LDS for each, and vals_out.  k: the thread's
+// keys, of blocks i * NT + thread (0: pinned or past the row).  False, with nothing done, when a bucket
+// is over the limit.
+template <int NT, int ITEMS, int MAX_ITEMS>
+__device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS], int open, int32_t *vals,
+                                             RowLds<NT, MAX_ITEMS> &lds) {
+  constexpr unsigned long long kZero = 1ull << 63;  // the key of a zero share; positive shares' are above it
+  const int lane = lane_id();
+  int tid = phase_thread();
+  unsigned long long top = 0ull, under = 0ull;  // the largest key, and the largest complement of one
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (k[i] > kZero) {
+      top = k[i] > top ? k[i] : top;
+      under = ~k[i] > under ? ~k[i] : under;
+    }
+  }
+  block_max2_u64<NT>(top, under, lds.scan64);
+  const unsigned long long bottom = ~under;
+  const unsigned long long span = top > bottom ? top - bottom : 0ull;
+  // coarse bin of x: x >> cut, at most kCoarse - 2
+  int cut = max(0, 64 - (int)__builtin_clzll(span | 1ull) - 9);
+  if ((span >> cut) >= kCoarse - 1) ++cut;
+  const int fixed = max(0, cut + kRowIndexBits - 64);  // bits a bucket has to fix for its words to hold the rest
+  if (fixed > 1) return false;                         // shares over more than 2^9 binades
+  for (int j = tid; j < kCoarse; j += NT) lds.coarse[j] = 0u;
+  for (int j = tid; j < lds.kBuckets / 2; j += NT) lds.bucket[j] = 0u;
+  for (int j = tid; j < (int)(sizeof(lds.heads) / 4); j += NT) lds.heads[j] = 0u;
+  if (tid == 0) lds.flag = 0;
+  lds_barrier();
+  tid = phase_thread();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if (k[i] != 0ull) atomicAdd(&lds.coarse[k[i] > kZero ? (int)((top - k[i]) >> cut) : kCoarse - 1], 1u);
+  lds_barrier();
+  tid = phase_thread();
+  {  // each bin's buckets: thread j takes bins j * kPer ..
+    constexpr int kPer = kCoarse > NT ? kCoarse / NT : 1;
+    int buckets[kPer], bits[kPer], mine = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int j = tid * kPer + q;
+      const int c = j < kCoarse ? (int)lds.coarse[j] : 0;
+      bits[q] = j == kCoarse - 1 ? 0 : min(cut, max(fixed, 30 - (int)__clz(max(c, 1))));
+      buckets[q] = c > 0 ? 1 << bits[q] : 0;
+      mine += buckets[q];
+    }
+    int all;
+    int at = block_exclusive_scan<NT, true>(mine, lds.scan, all);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int j = tid * kPer + q;
+      if (j < kCoarse) lds.coarse[j] = (unsigned int)at | ((unsigned int)bits[q] << 16);
+      at += buckets[q];
+    }
+  }
+  lds_barrier();
+  tid = phase_thread();
+  // a block's bucket, and its word: x's bits below the bucket's, then the block's index
+  auto place = [&](unsigned long long key, int b, int &bucket) {
+    const bool regular = key > kZero;
+    const unsigned long long x = top - key;
+    const unsigned int bin = lds.coarse[regular ? (int)(x >> cut) : kCoarse - 1];
+    const int low = cut - (int)(bin >> 16);  // the bits below the bucket's
+    const unsigned long long in_bin = x & ((1ull << cut) - 1ull);
+    bucket = (int)(bin & 0xffffu) + (regular ? (int)(in_bin >> low) : 0);
+    const unsigned long long rest = regular ? in_bin & ((1ull << low) - 1ull) : (key == kZero ? 0ull : 1ull);
+    return (rest << kRowIndexBits) | (unsigned long long)b;
+  };
+  uint32_t where[ITEMS];  // bucket | arrival << 16
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    where[i] = 0u;
+    if (k[i] != 0ull) {
+      int bucket;
+      place(k[i], 0, bucket);
+      const int half = 16 * (bucket & 1);
+      const unsigned int old = atomicAdd(&lds.bucket[bucket >> 1], 1u << half);
+      where[i] = (uint32_t)bucket | (((old >> half) & 0xffffu) << 16);
+    }
+    if (i % 4 == 3) keep_order();
+  }
+  lds_barrier();
+  tid = phase_thread();
+  {  // counts to first positions
+    constexpr int kWords = RowLds<NT, MAX_ITEMS>::kBuckets / 2;
+    constexpr int kPer = (kWords + NT - 1) / NT;
+    unsigned int w[kPer];
+    int mine = 0, most = 0;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int j = tid * kPer + q;
+      w[q] = j < kWords ? lds.bucket[j] : 0u;
+      const int a = (int)(w[q] & 0xffffu), b = (int)(w[q] >> 16);
+      mine += a + b;
+      most = max(most, max(a, b));
+    }
+    if (most > kBucketLimit) lds.flag = 1;
+    int all;
+    int at = block_exclusive_scan<NT, true>(mine, lds.scan, all);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      const int j = tid * kPer + q;
+      const int a = (int)(w[q] & 0xffffu), b = (int)(w[q] >> 16);
+      if (j < kWords) lds.bucket[j] = (unsigned int)at | ((unsigned int)(at + a) << 16);
+      if (a > 0) atomicOr(&lds.heads[at >> 5], 1u << (at & 31));
+      if (b > 0) atomicOr(&lds.heads[(at + a) >> 5], 1u << ((at + a) & 31));
+      at += a + b;
+    }
+  }
+  lds_barrier();
+  tid = phase_thread();
+  if (lds.flag != 0) return false;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (i % 4 == 0) keep_order();
+    if (k[i] != 0ull) {
+      int bucket;
+      const unsigned long long word = place(k[i], i * NT + tid, bucket);
+      const unsigned int first = lds.bucket[bucket >> 1] >> (16 * (bucket & 1)) & 0xffffu;
+      lds.elem[first + (where[i] >> 16)] = word;
+    }
+  }
+  lds_barrier();
+  tid = phase_thread();
+  // positions i * NT + thread: the bucket's bounds from the bitmap, then the blocks of it before this one
+  uint32_t moved[ITEMS];  // rank | index << 16
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int p0 = i * NT + tid - lane, p = p0 + lane;  // the wave's first position, a multiple of 64
+    moved[i] = 0u;
+    if (p0 < open) {
+      const int w0 = p0 >> 5;
+      const uint64_t here = (uint64_t)lds.heads[w0] | ((uint64_t)lds.heads[w0 + 1] << 32);
+      const uint64_t upto = here & (~0ull >> (63 - lane)), after = lane == 63 ? 0ull : here & (~0ull << (lane + 1));
+      int from, to;
+      if (upto != 0ull) {
+        from = p0 + 63 - __clzll((long long)upto);
+      } else {  // the bucket starts in an earlier word (position 0 is a head)
+        int w = w0 - 1;
+        while (w > 0 && lds.heads[w] == 0u) --w;
+        from = 32 * w + 31 - __clz((int)lds.heads[w]);
+      }
+      if (after != 0ull) {
+        to = p0 + __ffsll((long long)after) - 1;
+      } else {
+        int w = w0 + 2;
+        while (32 * w < open && lds.heads[w] == 0u) ++w;
+        to = 32 * w < open ? 32 * w + __ffs((int)lds.heads[w]) - 1 : open;
+      }
+      to = min(to, open);
+      if (p < open) {
+        const unsigned long long e = lds.elem[p];
+        int rank = from;
+        if (to - from > 1) {
+          for (int q = from; q < to; q += 4) {  // four reads in flight
+            unsigned long long x[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[c] = lds.elem[min(q + c, to - 1)];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) rank += q + c < to && x[c] < e ? 1 : 0;
+          }
+        }
+        moved[i] = (uint32_t)rank | ((uint32_t)(e & ((1ull << kRowIndexBits) - 1ull)) << 16);
+      }
+    }
+    keep_order();
+  }
+  lds_barrier();
+  tid = phase_thread();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (i * NT + tid < open) {
+      const int rank = (int)(moved[i] & 0xffffu), b = (int)(moved[i] >> 16);
+      vals[rank] = b;
+      lds.pos_of[b] = (unsigned short)rank;
+    }
+  }
+  lds_barrier();
+  return true;
+}
+
+// One window of a row's running totals: values pos .. of lds.share (K a thread) from the total t before
+// them, as scan_chunk's windows, but a tie does not end it: its rounding only adds 0 or 1 to the later
+// sums, so ties are first rounded down, then taken in order against the parity of the sum before each
+// (t / u's parity is its last bit), and the later sums raised by the ties that round up.  Returns the
+// values taken; those after them are as they were.  With more than kTies ties (TIES_END) the first one
+// ends the window instead.
+template <int K, bool TIES_END, int NT, int MAX_ITEMS>
+__device__ __forceinline__ int scan_window(int pos, int open, double t, RowLds<NT, MAX_ITEMS> &lds) {
+  const int tid = phase_thread(), lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint64_t tb = (uint64_t)__double_as_longlong(t);
+  const int eb = (int)(tb >> 52);  // t is a positive normal
+  const double u = __longlong_as_double((long long)((uint64_t)(eb - 52) << 52));      // 2^(E - 52)
+  const double inv = __longlong_as_double((long long)((uint64_t)(2098 - eb) << 52));  // 2^(52 - E)
+  const double room = 0x1p53 - t * inv;  // (2^(E+1) - t) / u, an integer
+  const int n = min(open - pos, K * NT), first = pos + tid * K;
+  double run[K], sum = 0.0;
+  uint32_t fits = 0u, ties = 0u;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int e = first + k;
+    const double y = lds.share[chunk_slot(min(e, open - 1))] * inv;  // every read issued, none under a condition
+    const bool in = e < pos + n && y >= 0.0 && y < 0x1p53;
+    const double r = __builtin_floor(y), f = y - r;
+    fits |= in && !(TIES_END && f == 0.5) ? 1u << k : 0u;
+    ties |= in && f == 0.5 ? 1u << k : 0u;
+    sum += in ? r + (f > 0.5 ? 1.0 : 0.0) : 0.0;
+    run[k] = sum;
+  }
+  // the values before this thread's: the lanes before it (the scan moved one lane up) and the waves
+  double before = wave_inclusive_scan_f64(dpp_move_f64<0x138, 0xf, true>(sum));
+  if (lane == kWave - 1) lds.wave_sum[wave] = before + sum;
+  if (threadIdx.x == 0) {
+    lds.stop = n;
+    lds.ties = 0;
+  }
+  lds_barrier();
+#pragma unroll
+  for (int w = 0; w < NT / kWave; ++w) before += w < wave ? lds.wave_sum[w] : 0.0;
+  if constexpr (!TIES_END) {
+    if (ties != 0u)
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        if ((ties >> k) & 1u) {
+          const int at = atomicAdd(&lds.ties, 1);
+          const double below = before + run[k];  // rounded down
+          if (at < kTies) lds.tie[at] = ((tid * K + k) << 1) | (below < 0x1p53 ? (int)((long long)below & 1) : 0);
+        }
+    lds_barrier();
+    const int count = lds.ties;
+    if (count > kTies) return -1;
+    if (count > 0) {
+      // every wave takes the ties in order: lane i the one with i before it
+      int mine = lane < count ? lds.tie[lane] : INT_MAX, rank = 0;
+      for (int i = 0; i < count; ++i) rank += __builtin_amdgcn_readlane(mine, i) < mine ? 1 : 0;
+      const int sorted = __builtin_amdgcn_ds_permute(4 * (lane < count ? rank : lane), mine);
+      int raised = (int)(tb & 1ull);  // t / u's parity, then the ties raised so far too
+      for (int i = 0; i < count; ++i) {
+        const int tie = __builtin_amdgcn_readlane(sorted, i);
+        if ((tie ^ raised) & 1) {
+          ++raised;
+          if ((tie >> 1) < tid * K) before += 1.0;
+          else
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+              if (tid * K + k >= (tie >> 1)) run[k] += 1.0;
+        }
+      }
+    }
+  }
+  int stop = K;
+#pragma unroll
+  for (int k = K - 1; k >= 0; --k) {
+    const double y = lds.share[chunk_slot(min(first + k, open - 1))] * inv;
+    const bool under = y < room - (before + (k > 0 ? run[k - 1] : 0.0));  // t + value < 2^(E+1)
+    if (!(((fits >> k) & 1u) && under)) stop = k;
+  }
+  const uint64_t stopped = __builtin_amdgcn_ballot_w64(stop < K);
+  if (stopped != 0ull) {
+    const int sl = __builtin_ctzll(stopped);
+    const int at = (wave * kWave + sl) * K + __builtin_amdgcn_readlane(stop, sl);
+    if (lane == 0) atomicMin(&lds.stop, at);
+  }
+  lds_barrier();
+  const int taken = lds.stop;  // at most the values left
+  const int local = taken - tid * K;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (k < local) lds.share[chunk_slot(first + k)] = t + (before + run[k]) * u;
+  lds_barrier();
+  return taken;
+}
+
+// The running totals of the request's sorted shares (lds.share, by chunk_slot), in place: see scan_chunk.
+// The value that ends a window takes its total by one addition.  The first values, and those after a
+// window that ended at once, are added one at a time by wave 0 (there the total crosses a binade every
+// few values); windows of two values a thread until one is taken whole, then eight.
+template <int NT, int MAX_ITEMS>
+__device__ __forceinline__ void scan_row(int open, RowLds<NT, MAX_ITEMS> &lds) {
+  double t = -0.0;
+  int pos = 0;
+  bool alone = true, wide = false;
+  while (pos < open) {
+    const int eb = (int)(((uint64_t)__double_as_longlong(t) >> 52) & 0x7ff);  // t's biased exponent
+    if (t != t) {                                                            // NaN: every later total is NaN
+      for (int e = pos + (int)threadIdx.x; e < open; e += NT) lds.share[chunk_slot(e)] = t;
+      break;
+    }
+    if (alone || !(t > 0.0) || eb < 63 || eb > 2022) {
+      const int run = min(open - pos, kWave);
+      if (threadIdx.x < kWave) {
+        // gathered in a line first: the chain's reads and writes then need no address arithmetic
+        const int lane = lane_id();
+        lds.line[lane] = lane < run ? lds.share[chunk_slot(pos + lane)] : -0.0;  // -0.0 changes no total
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k0 = 0; k0 < kWave; k0 += 16) {
+          double x[16];
+#pragma unroll
+          for (int k = 0; k < 16; ++k) x[k] = lds.line[k0 + k];
+#pragma unroll
+          for (int k = 0; k < 16; ++k) {
+            t += x[k];
+            x[k] = t;
+          }
+#pragma unroll
+          for (int k = 0; k < 16; ++k) lds.line[k0 + k] = x[k];
+        }
+        __builtin_amdgcn_wave_barrier();
+        const double total = lds.line[lane];
+        if (lane < run) lds.share[chunk_slot(pos + lane)] = total;
+      }
+      lds_barrier();
+      pos += run;
+      t = lds.share[chunk_slot(pos - 1)];
+      alone = false;
+      continue;
+    }
+    const int asked = min(open - pos, (wide ? 8 : 2) * NT);
+    int taken = wide ? scan_window<8, false, NT, MAX_ITEMS>(pos, open, t, lds)
+                     : scan_window<2, false, NT, MAX_ITEMS>(pos, open, t, lds);
+    if (taken < 0) {  // many ties
+      lds_barrier();
+      taken = scan_window<2, true, NT, MAX_ITEMS>(pos, open, t, lds);
+      alone = taken < min(open - pos, 2 * NT);
+    } else {
+      alone = taken < kWave;
+      wide = taken == asked;
+    }
+    if (taken > 0) t = lds.share[chunk_slot(pos + taken - 1)];
+    pos += taken;
+    if (pos < open && (taken < asked) && !alone) {
+      t += lds.share[chunk_slot(pos)];
+      lds_barrier();
+      if (threadIdx.x == 0) lds.share[chunk_slot(pos)] = t;
+      ++pos;
+    }
+  }
+  lds_barrier();
+}
+
+template <int NT, int ITEMS, int MAX_ITEMS>
+__device__ __forceinline__ void take_row(const MaxminParams &m, int r, int n, RowLds<NT, MAX_ITEMS> &lds) {
+  constexpr int kWaves = NT / kWave;
+  const Params &p = m.p;
+  const int lane = lane_id();
+  int tid = phase_thread();
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const double *srow = p.scores + (int64_t)r * p.scores_stride;
+  const bool masked = p.pinned != nullptr;
+  const uint8_t *prow = masked ? p.pinned + (int64_t)r * p.pinned_stride : reinterpret_cast<const uint8_t *>(srow);
+  RowStat st;
+  st.n = n;
+  // the blocks' keys; every load is unconditional and in range (n >= 1)
+  unsigned long long k[ITEMS];
+  uint32_t open_bits = 0u;
+  {
+    double score[ITEMS];
+    uint8_t pin[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int c = min(i * NT + tid, n - 1);
+      score[i] = srow[c];
+      pin[i] = prow[c];
+    }
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) lds.share[chunk_slot(i * NT + tid)] = clamp0(score[i]);
+    lds_barrier();
+    st.total = block_numpy_sum<NT, true>([&](int i) { return lds.share[chunk_slot(i)]; }, n, lds.pair);
+    const double first_share = share_value(st, lds.share[0]), last_share = share_value(st, lds.share[chunk_slot(n - 1)]);
+    lds_barrier();  // the scores are read before the list of the pinned shares
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int b = i * NT + tid;
+      k[i] = block_key(st, masked, b, score[i], pin[i]);
+      open_bits |= k[i] != 0ull ? 1u << i : 0u;
+      if (i % 4 == 3) keep_order();
+    }
+    // the pinned shares' sum
+    double base;
+    int pinned;
+    if (!masked) {
+      pinned = min(n, 2);
+      double sum = 0.0;
+      sum += first_share;
+      if (n >= 2) sum += last_share;
+      base = 0.0 + sum;  // base_default
+    } else {
+      // listed in block order in LDS: the pinned blocks of each 64 counted, scanned by wave 0, then placed
+      uint64_t mine = 0ull;
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) {
+        const uint64_t set = __ballot(i * NT + tid < n && !((open_bits >> i) & 1u));
+        if (lane == 0) lds.pin_count[i * kWaves + wave] = __popcll(set);
+      }
+      lds_barrier();
+      if (wave == 0) {
+        int carry = 0;
+        for (int j0 = 0; j0 < ITEMS * kWaves; j0 += kWave) {
+          const int c = j0 + lane < ITEMS * kWaves ? lds.pin_count[j0 + lane] : 0;
+          const int inc = wave_inclusive_scan(c);
+          if (j0 + lane < ITEMS * kWaves) lds.pin_count[j0 + lane] = carry + inc - c;
+          carry += __builtin_amdgcn_readlane(inc, kWave - 1);
+        }
+        if (lane == 0) lds.flag = carry;
+      }
+      lds_barrier();
+      pinned = lds.flag;
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) {
+        const bool pn = i * NT + tid < n && !((open_bits >> i) & 1u);
+        mine = __ballot(pn);
+        if (pn) {
+          const int at = lds.pin_count[i * kWaves + wave] +
+                         __builtin_amdgcn_mbcnt_hi((uint32_t)(mine >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mine, 0u));
+          lds.share[chunk_slot(at)] = share_value(st, score[i]);
+        }
+        keep_order();
+      }
+      lds_barrier();
+      base = block_numpy_sum<NT, true>([&](int i) { return lds.share[chunk_slot(i)]; }, pinned, lds.pair);
+    }
+    st.pinned = pinned;
+    st.open = n - pinned;
+    st.pad = 0;
+    if (tid == 0) {
+      lds.base = base;
+    }
+    lds_barrier();
+  }
+  const int open = st.open;
+  const int64_t row0 = (int64_t)r * p.width;
+  if (!bucket_ranks<NT, ITEMS, MAX_ITEMS>(k, open, m.vals_out + row0, lds)) {
+    radix_ranks<NT, ITEMS>(m, st, r, lds.elem, lds.count, &lds.flag);
+    uint32_t moved[ITEMS];
+    tid = phase_thread();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) moved[i] = (uint32_t)(lds.elem[i * NT + tid] & ((1ull << kIndexBits) - 1ull));
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int pos = i * NT + tid;
+      if (pos < n) {
+        m.vals_out[row0 + pos] = (int)moved[i];
+        lds.pos_of[moved[i]] = (unsigned short)pos;
+      }
+    }
+    // the keys again (not held across the sort)
+    tid = phase_thread();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int b = i * NT + tid, c = min(b, n - 1);
+      k[i] = block_key(st, masked, b, srow[c], prow[c]);
+      keep_order();
+    }
+    lds_barrier();
+  }
+  // the open shares in sorted order
+  tid = phase_thread();
+  uint32_t at[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) at[i] = lds.pos_of[i * NT + tid];
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if ((open_bits >> i) & 1u) lds.share[chunk_slot((int)at[i])] = key_value(k[i]);
+  lds_barrier();
+  scan_row<NT, MAX_ITEMS>(open, lds);
+  tid = phase_thread();
+  double *pre = m.prefix + row0;
+  for (int i = tid; i < open; i += NT) pre[i] = lds.share[chunk_slot(i)];
+  const double shift = 2.0 * (double)r, base = lds.base;
+  if (tid == 0) {
+    store_row_stat(p.row_stat + r, st);
+    m.mrow[r] = MaxminRow{base, open, 0};
+  }
+  // each level's position among the totals shifted by 2r, and its count (mm_totals_kernel)
+  constexpr int kMine = kLevels / NT;  // searched together, a step of each in flight
+  double need[kMine], target[kMine];
+  int lo[kMine], hi[kMine];
+#pragma unroll
+  for (int q = 0; q < kMine; ++q) {
+    need[q] = (double)(q * NT + tid) / kLevels - base;
+    target[q] = (need[q] - 1e-12) + shift;
+    lo[q] = 0;
+    hi[q] = open;
+  }
+  for (int step = 0; step < 32 - __clz(open); ++step) {  // an interval of n halves to at most n / 2
+#pragma unroll
+    for (int q = 0; q < kMine; ++q) {
+      const int mid = (lo[q] + hi[q]) >> 1;
+      const bool in = lo[q] < hi[q];
+      const bool up = lds.share[chunk_slot(in ? mid : 0)] + shift < target[q];
+      lo[q] = in && up ? mid + 1 : lo[q];
+      hi[q] = in && !up ? mid : hi[q];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kMine; ++q) {
+    const int j = q * NT + tid;
+    if (j > 0) {
+      set_pos(m, m.level_pos, r, j, lo[q]);
+      const int count = need[q] <= 1e-12 ? 0 : min(lo[q] + 1, open);
+      if (count > 0) atomicAdd(&m.level_count[j], count);
+    }
+  }
+}
+
+// One workgroup per request of at most NT * MAX_ITEMS blocks, the longest first.  The last workgroup to
+// arrive decides the budget's mode from every request's statistics (stored with device-coherent stores
+// that complete before a workgroup counts its arrival; the order kernel cleared the counter).
+template <int NT, int MAX_ITEMS>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4)))
+void mm_rows_kernel(const MaxminParams m) {
+  __shared__ RowLds<NT, MAX_ITEMS> lds;
+  const Params &p = m.p;
+  const int r = m.order[blockIdx.x];
+  const int n = row_blocks(p, r);
+  if (n <= 0) {
+    if (threadIdx.x == 0) {
+      store_row_stat(p.row_stat + r, RowStat{0.0, 0, 0, 0, 0});
+      m.mrow[r] = MaxminRow{0.0, 0, 0};
+    }
+    for (int j = threadIdx.x; j < kLevels; j += NT) set_pos(m, m.level_pos, r, j, 0);
+  } else if (MAX_ITEMS > 2 && n <= 2 * NT) {
+    take_row<NT, 2, MAX_ITEMS>(m, r, n, lds);
+  } else if (MAX_ITEMS > 4 && n <= 4 * NT) {
+    take_row<NT, MAX_ITEMS < 4 ? MAX_ITEMS : 4, MAX_ITEMS>(m, r, n, lds);
+  } else if (MAX_ITEMS > 8 && n <= 8 * NT) {
+    take_row<NT, MAX_ITEMS < 8 ? MAX_ITEMS : 8, MAX_ITEMS>(m, r, n, lds);
+  } else {
+    take_row<NT, MAX_ITEMS, MAX_ITEMS>(m, r, n, lds);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's stores have completed
+  __syncthreads();
+  if (threadIdx.x == 0)
+    lds.flag = __hip_atomic_fetch_add(&p.state->arrivals, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.rows - 1;
+  __syncthreads();
+  if (lds.flag) decide<NT, true>(p);
+}
+
+// Before mm_rows_kernel: the requests' order and the cleared level counts (order_requests), and the
+// arrival counter.
+__global__ __launch_bounds__(kSortThreads) void mm_order_kernel(const MaxminParams m) {
+  if (threadIdx.x == 0) m.p.state->arrivals = 0;
+  order_requests(m);
 }
 
 constexpr int kLevelThreads = 256;  // the second level-count pass's workgroups
@@ -2419,29 +3102,33 @@ namespace alloc {
 // The `maxmin` pipeline on prepared parameters (every workspace pointer in place).
 int launch_maxmin(MaxminParams m, int rows, int width, hipStream_t s) {
   Params &p = m.p;
-  hipLaunchKernelGGL(alloc::prepare_kernel, dim3(rows), dim3(alloc::kPrepThreads), 0, s, p);
-  const bool wide = width > alloc::kMaxWidth;
-  if (p.pinned == nullptr) {
-    hipLaunchKernelGGL(alloc::mm_plan_kernel<true>, dim3(1), dim3(alloc::kSortThreads), 0, s, m);
+  if (width <= alloc::kRowsWidth) {
+    hipLaunchKernelGGL(alloc::mm_order_kernel, dim3(1), dim3(alloc::kSortThreads), 0, s, m);
+    if (width <= 512) hipLaunchKernelGGL((alloc::mm_rows_kernel<256, 2>), dim3(rows), dim3(256), 0, s, m);
+    else if (width <= 1024) hipLaunchKernelGGL((alloc::mm_rows_kernel<256, 4>), dim3(rows), dim3(256), 0, s, m);
+    else if (width <= 4096) hipLaunchKernelGGL((alloc::mm_rows_kernel<512, 8>), dim3(rows), dim3(512), 0, s, m);
+    else hipLaunchKernelGGL((alloc::mm_rows_kernel<512, 16>), dim3(rows), dim3(512), 0, s, m);
+    const int rc = check_hip(hipGetLastError(), "ekv_rank_maxmin launch");
+    if (rc != EKV_OK) return rc;
   } else {
-    hipLaunchKernelGGL(alloc::mm_plan_kernel<false>, dim3(1), dim3(alloc::kSortThreads), 0, s, m);
-    if (wide) hipLaunchKernelGGL(alloc::mm_base_kernel<true>, dim3(rows), dim3(kWave), 0, s, m);
-    else hipLaunchKernelGGL(alloc::mm_base_kernel<false>, dim3(rows), dim3(kWave), 0, s, m);
+    hipLaunchKernelGGL(alloc::prepare_kernel, dim3(rows), dim3(alloc::kPrepThreads), 0, s, p);
+    const bool wide = width > alloc::kMaxWidth;
+    if (p.pinned == nullptr) {
+      hipLaunchKernelGGL(alloc::mm_plan_kernel<true>, dim3(1), dim3(alloc::kSortThreads), 0, s, m);
+    } else {
+      hipLaunchKernelGGL(alloc::mm_plan_kernel<false>, dim3(1), dim3(alloc::kSortThreads), 0, s, m);
+      if (wide) hipLaunchKernelGGL(alloc::mm_base_kernel<true>, dim3(rows), dim3(kWave), 0, s, m);
+      else hipLaunchKernelGGL(alloc::mm_base_kernel<false>, dim3(rows), dim3(kWave), 0, s, m);
+    }
+    int rc = check_hip(hipGetLastError(), "ekv_rank_maxmin launch");
+    if (rc != EKV_OK) return rc;
+    if (wide) hipLaunchKernelGGL(alloc::mm_wide_sort_kernel, dim3(rows), dim3(alloc::kSortThreads), 0, s, m);
+    else hipLaunchKernelGGL(alloc::mm_sort_kernel, dim3(rows), dim3(alloc::kSortThreads), 0, s, m);
+    rc = check_hip(hipGetLastError(), "ekv_rank_maxmin sort");
+    if (rc != EKV_OK) return rc;
+    hipLaunchKernelGGL(alloc::mm_totals_kernel, dim3((rows + alloc::kTotalsReqs - 1) / alloc::kTotalsReqs),
+                       dim3(alloc::kTotalsThreads), 0, s, m);
   }
-  int rc = check_hip(hipGetLastError(), "ekv_rank_maxmin launch");
-  if (rc != EKV_OK) return rc;
-  if (wide) {
-    hipLaunchKernelGGL(alloc::mm_wide_sort_kernel, dim3(rows), dim3(alloc::kSortThreads), 0, s, m);
-  } else if (width <= 4 * alloc::kSortThreads)
-    hipLaunchKernelGGL(alloc::mm_sort_kernel<4>, dim3(rows), dim3(alloc::kSortThreads), 0, s, m);
-  else if (width <= 8 * alloc::kSortThreads)
-    hipLaunchKernelGGL(alloc::mm_sort_kernel<8>, dim3(rows), dim3(alloc::kSortThreads), 0, s, m);
-  else
-    hipLaunchKernelGGL(alloc::mm_sort_kernel<12>, dim3(rows), dim3(alloc::kSortThreads), 0, s, m);
-  rc = check_hip(hipGetLastError(), "ekv_rank_maxmin sort");
-  if (rc != EKV_OK) return rc;
-  hipLaunchKernelGGL(alloc::mm_totals_kernel, dim3((rows + alloc::kTotalsReqs - 1) / alloc::kTotalsReqs),
-                     dim3(alloc::kTotalsThreads), 0, s, m);
   const dim3 level_grid((unsigned)std::min<int64_t>(rows, (int64_t)cu_count() * 2));
   hipLaunchKernelGGL(alloc::mm_levels2_kernel, level_grid, dim3(alloc::kLevelThreads), 0, s, m);
   if (rows > alloc::kMaxMaxminRegRows)

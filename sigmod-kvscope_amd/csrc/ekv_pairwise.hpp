@@ -119,7 +119,8 @@ __device__ double numpy_sum(Get get, int n, int *s_start, int *s_len, double *s_
 // the eight adds the leaf's last len % 8 values in order (all of a leaf shorter than 8, from 0.0).
 // The inner nodes then add their halves' sums, a level at a time from the deepest.  Each thread
 // loads the values of two leaves' accumulators before it adds any, so with NT = 256 a run of 8192
-// values costs one memory latency.  get(i) is also called for i = 0 when n is 0.  Contains barriers:
+// values costs one memory latency (IN_LDS: get reads LDS, and the values are added as they come, which
+// needs few registers).  get(i) is also called for i = 0 when n is 0.  Contains barriers:
 // every thread of the workgroup calls it.
 constexpr int kPairNodes = 1 << (kPairDepth + 1);  // heap slots 1 .. 255
 struct PairwiseLds {
@@ -128,10 +129,11 @@ struct PairwiseLds {
   int scan[16];
 };
 
-template <int NT, class Get>
+template <int NT, bool IN_LDS = false, class Get>
 __device__ double block_numpy_sum(Get get, int n, PairwiseLds &lds) {
   static_assert(NT % kWave == 0 && NT >= kPairNodes && NT <= 1024, "whole waves, a thread per tree node");
   constexpr int kPer = 16;  // values per accumulator in a leaf of at most 128
+  constexpr int H = NT >= 8 * 65 ? 1 : 2;  // chains a thread takes together (a run has at most 65 leaves)
   const int t = threadIdx.x, k = t & 7;
   const int v = t + 1;  // this thread's tree node (heap numbering), when v < kPairNodes
   const int depth = v < kPairNodes ? 31 - __clz(v) : 0;
@@ -165,11 +167,31 @@ __device__ double block_numpy_sum(Get get, int n, PairwiseLds &lds) {
     }
     lds_barrier();
     const int chains = 8 * leaves;  // a multiple of 8: the eight threads of a leaf go together
-    for (int c = t; c < chains; c += 2 * NT) {
-      double x[2][kPer], tail[2][7];
-      int m[2], rest[2];
+    if constexpr (IN_LDS) {
+      for (int c = t; c < chains; c += NT) {
+        const int s = lds.start[c >> 3], len = lds.len[c >> 3];
+        const int m = len >> 3;
+        double res = 0.0;
+        if (m > 0) {
+          double r = get(s + k);
+#pragma unroll 4
+          for (int i = 1; i < m; ++i) r += get(s + k + 8 * i);
+          r = r + __shfl_xor(r, 1, kWave);
+          r = r + __shfl_xor(r, 2, kWave);
+          r = r + __shfl_xor(r, 4, kWave);
+          res = r;
+        }
+        if (k == 0) {
+          for (int i = 8 * m; i < len; ++i) res += get(s + i);
+          lds.node[lds.node_of[c >> 3]] = res;
+        }
+      }
+    } else
+    for (int c = t; c < chains; c += H * NT) {
+      double x[H][kPer], tail[H][7];
+      int m[H], rest[H];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {  // chains c and c + NT: every load issued before any add
+      for (int h = 0; h < H; ++h) {  // chains c and c + NT: every load issued before any add
         const int cc = c + h * NT;
         const int j = cc < chains ? cc >> 3 : 0;
         const int s = lds.start[j], len = cc < chains ? lds.len[j] : 0;
@@ -190,7 +212,7 @@ __device__ double block_numpy_sum(Get get, int n, PairwiseLds &lds) {
         }
       }
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < H; ++h) {
         const int cc = c + h * NT;
         if (cc >= chains) continue;  // uniform over the eight threads of a leaf
         double res = 0.0;

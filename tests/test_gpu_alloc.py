@@ -257,6 +257,89 @@ def test_maxmin_running_totals_are_numpy_cumsums_bit_for_bit():
         assert got[fin].tobytes() == want[fin].tobytes(), (n, r % 6, int(np.argmax(got != want)))
 
 
+@pytest.mark.parametrize("width", [300, 512, 513, 1024, 1025, 3000, 4096, 4097, 8192])
+@pytest.mark.parametrize("masked", [False, True])
+def test_maxmin_rows_of_one_workgroup(width, masked):
+    # requests of at most 8192 blocks go from scores to running totals in one workgroup: ranks from
+    # buckets of the shares' leading bits, or a radix sort when a bucket is too full (equal shares,
+    # zeros) or the shares span more than 512 binades; totals in workgroup-wide windows.  Lengths at the
+    # edges of a thread's blocks, a wave and the row; the totals bit for bit np.cumsum's, the keep the
+    # oracle's (NaN and inf rows: the totals only)
+    rng = np.random.default_rng(900 + width + masked)
+    lengths = [n for n in (1, 2, 3, 63, 64, 65, 255, 257, 511, 600, 1023, 2047, 2049, 4095, 5000, 8191, width - 1,
+                           width, width, width, width, width, width, width, width // 2) if n <= width]
+    rows = len(lengths)
+    scores, pins = [], []
+    for r, n in enumerate(lengths):
+        kind = r % 8
+        if kind == 0:
+            x = rng.dirichlet(np.full(n, 0.1)).astype(np.float32).astype(np.float64)
+        elif kind == 1:
+            x = rng.integers(1, 9, size=n).astype(np.float64)
+        elif kind == 2:
+            x = rng.random(n) * 10.0 ** rng.uniform(-300, 0, size=n)
+        elif kind == 3:
+            x = rng.random(n)
+            x[rng.random(n) < 0.7] = 0.0
+        elif kind == 4:
+            x = rng.dirichlet(np.full(n, 10.0))
+        elif kind == 5:
+            x = 1.0 + rng.random(n) * 2.0 ** -30  # shares that differ in their low bits only
+        elif kind == 6:
+            x = np.repeat(rng.dirichlet(np.full(n, 0.3)), 2)[:n]
+        else:
+            x = np.where(rng.random(n) < 0.5, rng.random(n), 0.0)
+            x[: n // 100] = 0.0
+        scores.append(x)
+        if masked:
+            pin = rng.random(n) < rng.choice([0.0, 0.02, 0.5])
+            pin[0] = True
+            pins.append(pin)
+        else:
+            pins.append(oa.default_pins(n))
+    finite = rows
+    for special in (np.nan, np.inf):
+        x = rng.random(width)
+        x[width // 3] = special
+        scores.append(x)
+        lengths = lengths + [width]
+        pins.append(oa.default_pins(width))
+    for count, check_keep in ((finite, True), (finite + 2, False)):
+        grid = np.zeros((count, width))
+        mask = np.zeros((count, width), bool)
+        for r in range(count):
+            grid[r, : lengths[r]] = scores[r]
+            mask[r, : lengths[r]] = pins[r]
+        need = allocation.maxmin_workspace_bytes(count, width)
+        workspace = torch.zeros(need, dtype=torch.uint8, device="cuda")
+        total = sum(lengths[:count])
+        must = sum(int(p.sum()) for p in pins[:count])
+        budget = must + (total - must) // 2
+        keep, summary = allocation.maxmin_keep(
+            torch.from_numpy(grid).cuda(), torch.tensor(lengths[:count], dtype=torch.int32, device="cuda"),
+            budget=budget, pinned=torch.from_numpy(mask.astype(np.uint8)).cuda() if masked else None,
+            workspace=workspace)
+        assert summary.tolist()[:4] == [budget, total, must, 0]
+        raw = workspace.cpu().numpy()
+        cells = count * width * 8
+        prefix = (-workspace.data_ptr()) % 256 + need - 256 - (cells + 255) // 256 * 256
+        for r in range(count):
+            with np.errstate(invalid="ignore"):
+                sh = oa.shares(scores[r])  # inf / inf is NaN
+            open_sh = sh[~pins[r]]
+            nan = np.isnan(open_sh)
+            want = np.cumsum(np.concatenate([np.sort(open_sh[~nan])[::-1], open_sh[nan]]))
+            got = raw[prefix + r * width * 8: prefix + (r * width + len(want)) * 8].view(np.float64)
+            assert np.array_equal(np.isnan(got), np.isnan(want)), (lengths[r], r)
+            fin = ~np.isnan(want)
+            assert got[fin].tobytes() == want[fin].tobytes(), (lengths[r], r % 8)
+        if check_keep:
+            want = oa.allocate_maxmin(scores[:count], pins[:count], budget)
+            got = keep.cpu().numpy().astype(bool)
+            for r in range(count):
+                assert np.array_equal(got[r, : lengths[r]], want[r]), (lengths[r], r % 8)
+
+
 @pytest.mark.parametrize("seed", range(40))
 def test_maxmin_random_requests(seed):
     rng = np.random.default_rng(seed)
