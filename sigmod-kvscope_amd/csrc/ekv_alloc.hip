@@ -1459,8 +1459,8 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
 // sort, the running totals, and the positions of the levels j / kLevels in them.
 //
 // The sort places every open block by its exact rank, without passes over digits.  With x = (largest
-// key) - key, ascending in the sorted order, the blocks are counted in 511 coarse bins of x's leading
-// bits (zero and NaN shares in a bin of their own after them); a bin of c blocks is cut into about c / 2
+// key) - key, ascending in the sorted order, the blocks of positive shares are counted in 511 coarse bins
+// of x's leading bits (the zero shares follow in block order); a bin of c blocks is cut into about c / 2
 // to c / 4 buckets (two at least where the words below need it) of its next bits, so that a bucket holds a few blocks however the shares are spread;
 // and each block's rank is its bucket's first position plus the blocks of its bucket before it, counted
 // by comparing.  A bucket's bits fix all but x's low 51 bits (shares over more than 2^9 binades take the
@@ -1468,7 +1468,8 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
 // whole key and then the index: the order is the stable one whatever order the buckets were filled in.
 // Bucket bounds come from a bitmap of the buckets' first positions: a wave ranks 64 consecutive positions
 // and reads one word of it.  A request with a bucket of more than kBucketLimit blocks (many equal
-// shares, or shares that crowd together far below the bins' width) takes the radix sort instead.
+// shares, or shares that crowd together far below the bins' width) or a NaN share takes the radix sort
+// instead.
 //
 // The running totals are scan_chunk's exact windows over the whole workgroup, in which only a new binade
 // ends a window (scan_window), so a long request takes ~5 windows.
@@ -1481,7 +1482,7 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
 // VGPRs spilled (328 us); __syncthreads' waits for global stores cost ~5 us a request.
 constexpr int kRowsWidth = 8 * kSortThreads;  // the widest request
 static_assert(kRowsWidth <= 1 << 13, "a block index fits a bucket sort's word");
-constexpr int kCoarse = 512;                  // coarse bins; the last one holds the zero and NaN shares
+constexpr int kCoarse = 512;                  // coarse bins
 constexpr int kBucketLimit = 128;
 constexpr int kTies = 64;  // ties of a scan window resolved in place
 constexpr int kRowIndexBits = 13;             // block indices in a bucket sort's words
@@ -1521,6 +1522,7 @@ struct RowLds {
   };
   double base;
   int flag, stop, ties, tie[kTies];
+  unsigned short zero_count[NT / kWave * ITEMS];
 };
 
 // Keeps the compiler from interleaving one block's work with the next one's (eight blocks' at once spill).
@@ -1590,9 +1592,25 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
   tid = phase_thread();
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i)
-    if (k[i] != 0ull) atomicAdd(&lds.coarse[k[i] > kZero ? (int)((top - k[i]) >> cut) : kCoarse - 1], 1u);
+  {
+    if (k[i] > kZero) atomicAdd(&lds.coarse[(int)((top - k[i]) >> cut)], 1u);
+    const uint64_t zeros = __ballot(k[i] == kZero);
+    if (lane == 0) lds.zero_count[i * (NT / kWave) + (tid / kWave)] = (unsigned short)__popcll(zeros);
+    if (k[i] == 1ull) lds.flag = 1;  // NaN
+  }
   lds_barrier();
   tid = phase_thread();
+  if (tid < kWave) {  // the zero shares before each 64 blocks
+    int carry = 0;
+    for (int j0 = 0; j0 < ITEMS * (NT / kWave); j0 += kWave) {
+      const bool in = j0 + lane < ITEMS * (NT / kWave);
+      const int c = in ? lds.zero_count[j0 + lane] : 0;
+      const int inc = wave_inclusive_scan(c);
+      if (in) lds.zero_count[j0 + lane] = (unsigned short)(carry + inc - c);
+      carry += __builtin_amdgcn_readlane(inc, kWave - 1);
+    }
+    if (lane == 0) lds.stop = carry;
+  }
   {  // each bin's buckets: thread j takes bins j * kPer ..
     constexpr int kPer = kCoarse > NT ? kCoarse / NT : 1;
     int buckets[kPer], bits[kPer], mine = 0;
@@ -1600,7 +1618,7 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
     for (int q = 0; q < kPer; ++q) {
       const int j = tid * kPer + q;
       const int c = j < kCoarse ? (int)lds.coarse[j] : 0;
-      bits[q] = j == kCoarse - 1 ? 0 : min(cut, max(fixed, 30 - (int)__clz(max(c, 1))));
+      bits[q] = min(cut, max(fixed, 30 - (int)__clz(max(c, 1))));
       buckets[q] = c > 0 ? 1 << bits[q] : 0;
       mine += buckets[q];
     }
@@ -1617,20 +1635,19 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
   tid = phase_thread();
   // a block's bucket, and its word: x's bits below the bucket's, then the block's index
   auto place = [&](unsigned long long key, int b, int &bucket) {
-    const bool regular = key > kZero;
     const unsigned long long x = top - key;
-    const unsigned int bin = lds.coarse[regular ? (int)(x >> cut) : kCoarse - 1];
+    const unsigned int bin = lds.coarse[(int)(x >> cut)];
     const int low = cut - (int)(bin >> 16);  // the bits below the bucket's
     const unsigned long long in_bin = x & ((1ull << cut) - 1ull);
-    bucket = (int)(bin & 0xffffu) + (regular ? (int)(in_bin >> low) : 0);
-    const unsigned long long rest = regular ? in_bin & ((1ull << low) - 1ull) : (key == kZero ? 0ull : 1ull);
+    bucket = (int)(bin & 0xffffu) + (int)(in_bin >> low);
+    const unsigned long long rest = in_bin & ((1ull << low) - 1ull);
     return (rest << kRowIndexBits) | (unsigned long long)b;
   };
   uint32_t where[ITEMS];  // bucket | arrival << 16
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     where[i] = 0u;
-    if (k[i] != 0ull) {
+    if (k[i] > kZero) {
       int bucket;
       place(k[i], 0, bucket);
       const int half = 16 * (bucket & 1);
@@ -1673,7 +1690,7 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     if (i % 4 == 0) keep_order();
-    if (k[i] != 0ull) {
+    if (k[i] > kZero) {
       int bucket;
       const unsigned long long word = place(k[i], i * NT + tid, bucket);
       const unsigned int first = lds.bucket[bucket >> 1] >> (16 * (bucket & 1)) & 0xffffu;
@@ -1682,13 +1699,14 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
   }
   lds_barrier();
   tid = phase_thread();
+  const int positive = open - lds.stop;  // the zero shares follow in block order
   // positions i * NT + thread: the bucket's bounds from the bitmap, then the blocks of it before this one
   uint32_t moved[ITEMS];  // rank | index << 16
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     const int p0 = i * NT + tid - lane, p = p0 + lane;  // the wave's first position, a multiple of 64
     moved[i] = 0u;
-    if (p0 < open) {
+    if (p0 < positive) {
       const int w0 = p0 >> 5;
       const uint64_t here = (uint64_t)lds.heads[w0] | ((uint64_t)lds.heads[w0 + 1] << 32);
       const uint64_t upto = here & (~0ull >> (63 - lane)), after = lane == 63 ? 0ull : here & (~0ull << (lane + 1));
@@ -1704,11 +1722,11 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
         to = p0 + __ffsll((long long)after) - 1;
       } else {
         int w = w0 + 2;
-        while (32 * w < open && lds.heads[w] == 0u) ++w;
-        to = 32 * w < open ? 32 * w + __ffs((int)lds.heads[w]) - 1 : open;
+        while (32 * w < positive && lds.heads[w] == 0u) ++w;
+        to = 32 * w < positive ? 32 * w + __ffs((int)lds.heads[w]) - 1 : positive;
       }
-      to = min(to, open);
-      if (p < open) {
+      to = min(to, positive);
+      if (p < positive) {
         const unsigned long long e = lds.elem[p];
         int rank = from;
         if (to - from > 1) {
@@ -1729,10 +1747,17 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
   tid = phase_thread();
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
-    if (i * NT + tid < open) {
+    if (i * NT + tid < positive) {
       const int rank = (int)(moved[i] & 0xffffu), b = (int)(moved[i] >> 16);
       vals[rank] = b;
       lds.pos_of[b] = (unsigned short)rank;
+    }
+    const uint64_t zeros = __ballot(k[i] == kZero);
+    if (k[i] == kZero) {
+      const int rank = positive + lds.zero_count[i * (NT / kWave) + tid / kWave] +
+                       __builtin_amdgcn_mbcnt_hi((uint32_t)(zeros >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)zeros, 0u));
+      vals[rank] = i * NT + tid;
+      lds.pos_of[i * NT + tid] = (unsigned short)rank;
     }
   }
   lds_barrier();
