@@ -193,18 +193,30 @@ def check(status: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call entry point ``name`` and raise on a non-zero status."""
-    check(getattr(load(), name)(*args), name)
+    status = getattr(_lib or load(), name)(*args)
+    if status != OK:
+        check(status, name)
+
+
+_raw_stream = None  # torch's raw handle of a device's current stream, once torch's CUDA part is up
 
 
 def stream_handle(stream=None) -> int:
     """The raw hipStream_t of ``stream``: a torch stream, a raw handle (int) as is, or by default
-    torch's current stream on the current device."""
-    if isinstance(stream, int):
-        return stream
+    torch's current stream on the current device (read without building a stream object, ~0.4 us
+    against ~3 us)."""
+    global _raw_stream
+    if stream is not None:
+        return stream if isinstance(stream, int) else int(stream.cuda_stream)
+    if _raw_stream is not None:
+        return _raw_stream[0](_raw_stream[1]())
     import torch
 
-    s = torch.cuda.current_stream() if stream is None else stream
-    return int(s.cuda_stream)
+    current = int(torch.cuda.current_stream().cuda_stream)  # initialises CUDA
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None:
+        _raw_stream = (raw, torch.cuda.current_device)
+    return current
 
 
 def malloc(nbytes: int) -> int:
@@ -251,17 +263,22 @@ def synchronize() -> None:
     call("ekv_synchronize")
 
 
+_codes: dict = {}  # torch dtype -> EKV_* code
+
+
 def dtype_code(dtype) -> int:
     """The EKV_* element-type code of a torch dtype."""
-    import torch
+    if not _codes:
+        import torch
 
-    codes = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
-    fp8 = getattr(torch, "float8_e4m3fn", None)
-    if fp8 is not None:
-        codes[fp8] = FP8_E4M3
-    if dtype not in codes:
+        _codes.update({torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16})
+        fp8 = getattr(torch, "float8_e4m3fn", None)
+        if fp8 is not None:
+            _codes[fp8] = FP8_E4M3
+    code = _codes.get(dtype)
+    if code is None:
         raise ValueError(f"unsupported element type {dtype}")
-    return codes[dtype]
+    return code
 
 
 def ptr(tensor) -> int:

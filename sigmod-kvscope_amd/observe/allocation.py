@@ -40,6 +40,17 @@ def check_tensors(*specs) -> torch.device | None:
     """Refuse, with ValueError, tensors a kernel would misread.  ``specs`` are ``(name, tensor, dtypes,
     shape)``, ``tensor`` None for an absent optional one.  Every tensor's shape, dtype and row
     contiguity are checked first, then that all are on one GPU; returns that device."""
+    device = None
+    for _, t, dtypes, shape in specs:  # the sound call: one look at each tensor
+        if t is None:
+            continue
+        if not (isinstance(t, torch.Tensor) and t.shape == tuple(shape) and t.is_cuda
+                and (t.dtype in dtypes if isinstance(dtypes, tuple) else t.dtype == dtypes)
+                and (not shape or t.stride(-1) == 1) and (device is None or t.device == device)):
+            break
+        device = t.device
+    else:
+        return device
     present = [(name, t, dtypes, shape) for name, t, dtypes, shape in specs if t is not None]
     for name, t, dtypes, shape in present:
         if not isinstance(t, torch.Tensor):
@@ -59,6 +70,13 @@ def check_tensors(*specs) -> torch.device | None:
         elif t.device != device:
             raise ValueError(f"{name} is on {t.device}, the others on {device}")
     return device
+
+
+def new_summary(rows: int, device) -> torch.Tensor:
+    """The six int64 numbers a ranking writes: every kernel writes all of them, so nothing clears them
+    first (a fill is a launch of its own), but a call with no rows launches none."""
+    make = torch.empty if rows else torch.zeros
+    return make(6, dtype=torch.int64, device=device)
 
 
 def _out(out: torch.Tensor | None, rows: int, width: int, device) -> torch.Tensor:
@@ -183,7 +201,7 @@ def maxmin_keep(
     if budget < 0:
         raise ValueError("the budget cannot be negative")
     out = _out(out, rows, width, dev)
-    summary = torch.zeros(6, dtype=torch.int64, device=dev)
+    summary = new_summary(rows, dev)
     need = maxmin_workspace_bytes(rows, width)
     workspace = _workspace("workspace", workspace, need, dev)
     ekv_hip.call(
@@ -230,7 +248,7 @@ def sum_keep(
     if budget < 0:
         raise ValueError("the budget cannot be negative")
     out = _out(out, rows, width, dev)
-    summary = torch.zeros(6, dtype=torch.int64, device=dev)
+    summary = new_summary(rows, dev)
     need = sum_workspace_bytes(rows)
     workspace = _workspace("workspace", workspace, need, dev)
     ekv_hip.call(
@@ -279,7 +297,7 @@ def uniform_keep(
                         ("released", released, _MASK_DTYPES, (rows, width)),
                         ("pin_from", pin_from, torch.int32, (rows,)))
     out = _out(out, rows, width, dev)
-    summary = torch.zeros(6, dtype=torch.int64, device=dev)
+    summary = new_summary(rows, dev)
     wide = scores.dtype == torch.float64
     need = uniform_workspace_bytes(rows, scores.dtype) if (wide or pinned is not None or released is not None) else 0
     ws = _workspace("workspace", workspace, need, dev) if need else None

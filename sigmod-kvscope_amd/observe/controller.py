@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 
 import ekv_hip
-from observe.allocation import _MASK_DTYPES, Objective, _workspace, check_tensors, uniform_keep
+from observe.allocation import _MASK_DTYPES, Objective, _workspace, check_tensors, new_summary, uniform_keep
 
 _OBJECTIVE_CODES = {"sum": ekv_hip.OBJ_SUM, "maxmin": ekv_hip.OBJ_MAXMIN}
 
@@ -72,7 +72,7 @@ def keep_rows(
         out = torch.empty(rows, width, dtype=torch.uint8, device=dev)
     elif check_tensors(("out", out, torch.uint8, (rows, width))) != dev:
         raise ValueError(f"out must be on {dev}")
-    summary = torch.zeros(6, dtype=torch.int64, device=dev)
+    summary = new_summary(rows, dev)
     code = _OBJECTIVE_CODES[objective]
     ws = _workspace("workspace", workspace, keep_rows_workspace_bytes(objective, rows, width), dev)
     ekv_hip.call(

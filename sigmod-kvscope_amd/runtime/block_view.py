@@ -27,7 +27,7 @@ import numpy as np
 import torch
 
 import ekv_hip
-from observe.allocation import check_tensors
+from observe.allocation import check_tensors, new_summary
 from runtime.audit import AuditPlane
 
 
@@ -101,7 +101,7 @@ def uniform_view(
     if counts is not None and not counts.is_contiguous():
         raise ValueError("counts must be a contiguous int64 [rows, 5] tensor")
     keep = torch.empty(rows, width, dtype=torch.uint8, device=scores.device)
-    summary = torch.zeros(6, dtype=torch.int64, device=scores.device)
+    summary = new_summary(rows, scores.device)
     view = torch.empty(rows, width, dtype=torch.int32, device=table.device)
     lens = torch.empty(rows, dtype=torch.int32, device=table.device)
     ekv_hip.call(
@@ -355,15 +355,16 @@ class DecodeView:
         n = len(query_lens)
         q = np.asarray(query_lens.numpy() if isinstance(query_lens, torch.Tensor) else query_lens)
         decode = q == 1
-        servable = decode | (self.final_prefill[:n] & self.prefill_audit)
+        prefilled = self.final_prefill
         self.final_prefill = np.zeros(self.rows, dtype=bool)
         audited = np.zeros(self.rows, dtype=bool)
-        audited[:n] = self._state.wants_audit[:n] & servable
-        if audited.any() and not self.may_audit():
-            audited[:] = False  # the controller has not read the last audit yet
-        if (audited[:n] & ~decode).any() and self.on_prefill_audit is not None:
-            self.on_prefill_audit()
-        self._state.wants_audit[audited] = False
+        if self._state.wants_audit[:n].any():  # most steps audit nothing
+            audited[:n] = self._state.wants_audit[:n] & (decode | (prefilled[:n] & self.prefill_audit))
+            if audited.any() and not self.may_audit():
+                audited[:] = False  # the controller has not read the last audit yet
+            if (audited[:n] & ~decode).any() and self.on_prefill_audit is not None:
+                self.on_prefill_audit()
+            self._state.wants_audit[audited] = False
         self.audit_step = bool(audited.any())
         if self.audit_step:
             self._pending = audited
