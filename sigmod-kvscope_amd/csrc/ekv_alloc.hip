@@ -1474,7 +1474,7 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
 // The running totals are scan_chunk's exact windows over the whole workgroup, in which only a new binade
 // ends a window (scan_window), so a long request takes ~5 windows.
 //
-// At 1024 x U[1, 8192]: 112 us, where the totals, the radix sort of every request and a scan wave and a
+// At 1024 x U[1, 8192]: 115 us, where the totals, the radix sort of every request and a scan wave and a
 // level wave a request took 12 + 99 + 55; at 128 x U[32, 512]: 17 us for 6 + 12 + 25.  Bound by a
 // request's chain of phases, each a few LDS round trips and dependent float64 operations between
 // barriers (~120000 cycles for 8192 blocks: loads 15, total 7, keys 7, ranks 45, totals 25, levels 7),
