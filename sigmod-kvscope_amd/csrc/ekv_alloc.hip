@@ -393,17 +393,37 @@ constexpr int kCandPerRow = 1024;  // the list's room per request row
 // workgroup are serialised in memory, so fewer, larger workgroups end the pass sooner.
 constexpr int kHistThreads = 1024;
 
-// Workgroup w of a pass takes rows w, w + grid, ...: its region of the list holds kCandPerRow pairs
-// for each of them, after the regions of the workgroups before it.
+// A row of a pass is SPAN threads', so a workgroup takes kHistThreads / SPAN rows side by side: worker v
+// (threads SPAN (v mod that many) .. of workgroup v / that many) takes rows v, v + all workers, ....  Many
+// short rows then fill a workgroup, and there are fewer histograms to add up.
+template <int SPAN>
+struct PassRows {
+  static constexpr int kSide = kHistThreads / SPAN;  // rows side by side
+  __device__ static __forceinline__ int worker() { return (int)blockIdx.x * kSide + (int)threadIdx.x / SPAN; }
+  __device__ static __forceinline__ int stride() { return (int)gridDim.x * kSide; }
+};
+// The threads of a row, and the passes' workgroups.  An eighth of the width covers a row, but fewer than
+// ~32 workgroups lose more than they save: calls of 911 x 299 blocks take 67 us at 64 threads a row (90 at
+// 1024), 323 x 247 76 at 256 (93 at 1024), 128 x 512 with masks 50 at 256, 54 at 64 (8 workgroups) and 51 at
+// 1024, 14 x 1979 39 at 1024 and 42 at 256.
+inline int pass_span(int rows, int width) {
+  if (width <= 64 * kRun && rows >= 512) return 64;
+  return width <= 256 * kRun && rows >= 128 ? 256 : kHistThreads;
+}
+inline int pass_grid(int rows, int width, int cus) {
+  const int side = kHistThreads / pass_span(rows, width);
+  return std::min((rows + side - 1) / side, cus);
+}
+
+// Workgroup w's region of the list: an equal share of the list's kCandPerRow pairs a row.
 __device__ __forceinline__ void cand_region(int rows, int w, int grid, long long &first, int &room) {
-  const int per = rows / grid, extra = rows % grid;
-  first = (long long)kCandPerRow * ((long long)w * per + min(w, extra));
-  room = kCandPerRow * (per + (w < extra ? 1 : 0));
+  room = (int)((long long)kCandPerRow * rows / grid);
+  first = (long long)room * w;
 }
 
 constexpr int kHistRows = 2;  // rows whose blocks a pass's workgroup loads together
 
-template <bool TIE, int CAND_MODE, bool PIN>
+template <bool TIE, int CAND_MODE, bool PIN, int SPAN>
 __global__ __launch_bounds__(kHistThreads) void hist_kernel(const Params p, int shift, int bits, int last_gain_pass) {
   constexpr int cand_mode = CAND_MODE;
   __shared__ unsigned int s_hist[kBins];
@@ -462,8 +482,8 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const Params p, int 
     // writes the keep of every block the first digit decides (pinned and past-the-row blocks 1, an
     // open block 1 or 0 as its digit is above or below the threshold's), across the whole width, and
     // leaves the blocks it lists to the keep kernel.
-    const int G = gridDim.x;
-    for (int r0 = blockIdx.x; r0 < p.rows; r0 += kHistRows * G) {
+    const int G = PassRows<SPAN>::stride(), t = threadIdx.x % SPAN;
+    for (int r0 = __builtin_amdgcn_readfirstlane(PassRows<SPAN>::worker()); r0 < p.rows; r0 += kHistRows * G) {
       int rr[kHistRows], nmax = 0;
       RowStat st[kHistRows];
       double weight[kHistRows];
@@ -477,15 +497,15 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const Params p, int 
         nmax = max(nmax, st[i].n);
       }
       const int steps_to = cand_mode == 1 ? p.width : nmax;
-      for (int c0 = 0; c0 < steps_to; c0 += kHistThreads * kRun) {
-        BlockRun<kRun, kHistThreads, PIN> run[kHistRows];
+      for (int c0 = 0; c0 < steps_to; c0 += SPAN * kRun) {
+        BlockRun<kRun, SPAN, PIN> run[kHistRows];
 #pragma unroll
-        for (int i = 0; i < kHistRows; ++i) run[i].load(p, rr[i], c0 + threadIdx.x, st[i].n);
+        for (int i = 0; i < kHistRows; ++i) run[i].load(p, rr[i], c0 + t, st[i].n);
 #pragma unroll
         for (int i = 0; i < kHistRows; ++i) {
 #pragma unroll
           for (int u = 0; u < kRun; ++u) {
-            const int b = c0 + threadIdx.x + u * kHistThreads;
+            const int b = c0 + t + u * SPAN;
             bool counted = false;
             unsigned int digit = 0u;
             unsigned long long k = 0ull;
@@ -539,7 +559,7 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const Params p, int 
 // the blocks it listed, and a workgroup writes its list's; otherwise (another mode, an error, a
 // select that ended at the first pass) or when its list outgrew its room, the workgroup writes every
 // block of its rows.
-template <bool PIN>
+template <bool PIN, int SPAN>
 __global__ __launch_bounds__(kHistThreads) void sum_keep_kernel(const Params p) {
   const State *s = p.state;
   const int mode = s->mode;
@@ -565,16 +585,17 @@ __global__ __launch_bounds__(kHistThreads) void sum_keep_kernel(const Params p) 
     }
     return;
   }
-  for (int r = blockIdx.x; r < p.rows; r += gridDim.x) {
+  const int t = threadIdx.x % SPAN;
+  for (int r = PassRows<SPAN>::worker(); r < p.rows; r += PassRows<SPAN>::stride()) {
     const RowStat st = p.row_stat[r];
     const double weight = weight_of(p, r);
     uint8_t *krow = p.keep + (int64_t)r * p.keep_stride;
-    for (int b0 = threadIdx.x; b0 - (int)threadIdx.x < p.width; b0 += kHistThreads * kRun) {
-      BlockRun<kRun, kHistThreads, PIN> run;
+    for (int b0 = t; b0 - t < p.width; b0 += SPAN * kRun) {
+      BlockRun<kRun, SPAN, PIN> run;
       run.load(p, r, b0, st.n);
 #pragma unroll
       for (int u = 0; u < kRun; ++u) {
-        const int b = b0 + u * kHistThreads;
+        const int b = b0 + u * SPAN;
         if (b >= p.width) continue;
         uint8_t k;
         if (error || b >= st.n || mode == kKeepAll || ((run.pinned >> u) & 1u)) k = 1;
@@ -2972,31 +2993,39 @@ int launch_sum(Params p, hipStream_t s) {
   p.tie_rbits = tie_request_bits(rows);
   hipLaunchKernelGGL(alloc::prepare_kernel, dim3(rows), dim3(alloc::kPrepThreads), 0, s, p);
   hipLaunchKernelGGL(alloc::decide_kernel, dim3(1), dim3(alloc::kThreads), 0, s, p);
-  const dim3 grid((unsigned)std::min<int64_t>(rows, (int64_t)cu_count()));
-  // the gain threshold, kDigitBits at a time from the top of the 64-bit key
-  // (the second pass lists the blocks in the first pass's bucket; the later passes read that list)
-  // the kernels for the caller's pins: a mask, or each row's first and last block
-  const bool pin = p.pinned != nullptr;
-  using Pass = void (*)(alloc::Params, int, int, int);
-  const Pass first = pin ? alloc::hist_kernel<false, 0, true> : alloc::hist_kernel<false, 0, false>;
-  const Pass second = pin ? alloc::hist_kernel<false, 1, true> : alloc::hist_kernel<false, 1, false>;
-  const Pass listed = pin ? alloc::hist_kernel<false, 2, true> : alloc::hist_kernel<false, 2, false>;
-  const Pass tied = pin ? alloc::hist_kernel<true, 2, true> : alloc::hist_kernel<true, 2, false>;
-  int pass = 0;
-  for (int top = 64; top > 0; top -= alloc::kDigitBits, ++pass) {
-    const int shift = std::max(top - alloc::kDigitBits, 0), bits = top - shift;
-    const int last = shift == 0 ? 1 : 0;
-    const Pass kernel = pass == 0 ? first : pass == 1 ? second : listed;
-    hipLaunchKernelGGL(kernel, grid, dim3(alloc::kHistThreads), 0, s, p, shift, bits, last);
-  }
-  // among the blocks at the threshold: newer block, earlier request (the tie key)
-  static_assert(alloc::kMaxSumWidth <= (1 << 18), "the tie key's block field is at most 18 bits");
-  for (int top = tie_bits(p.width, p.tie_rbits); top > 0; top -= alloc::kDigitBits) {
-    const int shift = std::max(top - alloc::kDigitBits, 0), bits = top - shift;
-    hipLaunchKernelGGL(tied, grid, dim3(alloc::kHistThreads), 0, s, p, shift, bits, -1);
-  }
-  hipLaunchKernelGGL(pin ? alloc::sum_keep_kernel<true> : alloc::sum_keep_kernel<false>, grid,
-                     dim3(alloc::kHistThreads), 0, s, p);
+  const dim3 grid((unsigned)pass_grid(rows, p.width, cu_count()));
+  static_assert(kMaxSumWidth <= (1 << 18), "the tie key's block field is at most 18 bits");
+  // the kernels for the caller's pins (a mask, or each row's first and last block) and rows
+  auto passes = [&](auto pin_tag, auto span_tag) {
+    constexpr bool PIN = decltype(pin_tag)::value;
+    constexpr int SPAN = decltype(span_tag)::value;
+    const dim3 block(kHistThreads);
+    // the gain threshold, kDigitBits at a time from the top of the 64-bit key
+    // (the second pass lists the blocks in the first pass's bucket; the later passes read that list)
+    int pass = 0;
+    for (int top = 64; top > 0; top -= kDigitBits, ++pass) {
+      const int shift = std::max(top - kDigitBits, 0), bits = top - shift;
+      const int last = shift == 0 ? 1 : 0;
+      if (pass == 0) hipLaunchKernelGGL((hist_kernel<false, 0, PIN, SPAN>), grid, block, 0, s, p, shift, bits, last);
+      else if (pass == 1) hipLaunchKernelGGL((hist_kernel<false, 1, PIN, SPAN>), grid, block, 0, s, p, shift, bits, last);
+      else hipLaunchKernelGGL((hist_kernel<false, 2, PIN, SPAN>), grid, block, 0, s, p, shift, bits, last);
+    }
+    // among the blocks at the threshold: newer block, earlier request (the tie key)
+    for (int top = tie_bits(p.width, p.tie_rbits); top > 0; top -= kDigitBits) {
+      const int shift = std::max(top - kDigitBits, 0), bits = top - shift;
+      hipLaunchKernelGGL((hist_kernel<true, 2, PIN, SPAN>), grid, block, 0, s, p, shift, bits, -1);
+    }
+    hipLaunchKernelGGL((sum_keep_kernel<PIN, SPAN>), grid, block, 0, s, p);
+  };
+  auto spans = [&](auto pin_tag) {
+    switch (pass_span(rows, p.width)) {
+      case 64: passes(pin_tag, std::integral_constant<int, 64>()); break;
+      case 256: passes(pin_tag, std::integral_constant<int, 256>()); break;
+      default: passes(pin_tag, std::integral_constant<int, kHistThreads>()); break;
+    }
+  };
+  if (p.pinned != nullptr) spans(std::true_type());
+  else spans(std::false_type());
   return check_hip(hipGetLastError(), "ekv_rank_sum launch");
 }
 

@@ -188,6 +188,35 @@ def test_maxmin_more_than_65536_requests():
     assert bad == 0 and int(summary[4]) == rows
 
 
+@pytest.mark.parametrize("rows,width", [(127, 300), (128, 512), (129, 513), (130, 2048), (131, 2049), (511, 40),
+                                        (512, 512), (513, 511), (700, 513), (1025, 64)])
+@pytest.mark.parametrize("kind", ["shares", "ties"])
+def test_sum_rows_side_by_side(rows, width, kind):
+    # the passes take a row with 64, 256 or 1024 threads by the number of rows and the width: both sides of
+    # each line, with lists that hold (shares) and that outgrow their room (many equal gains), pins and
+    # weights, strided keeps; whole numbers, so equal to the oracle's
+    rng = np.random.default_rng(700 + rows + width)
+    sizes = rng.integers(0, width + 1, size=rows)
+    sizes[0] = width
+    scores = rng.gamma(0.1, size=(rows, width)) if kind == "shares" else rng.integers(0, 2, (rows, width)).astype(float)
+    pins = rng.random((rows, width)) < 0.05
+    weights = rng.uniform(0.5, 2.0, size=rows) if kind == "shares" else np.ones(rows)
+    must, total = int(sum(pins[r, : sizes[r]].sum() for r in range(rows))), int(sizes.sum())
+    budget = must + (total - must) // 2
+    out = torch.full((rows, width + 5), 7, dtype=torch.uint8, device="cuda")
+    keep, summary = allocation.sum_keep(
+        torch.from_numpy(scores).cuda(), torch.from_numpy(sizes.astype(np.int32)).cuda(), budget=budget,
+        weights=torch.from_numpy(weights).cuda(), pinned=torch.from_numpy(pins.astype(np.uint8)).cuda(),
+        out=out[:, :width])
+    want = oa.allocate_sum([scores[r, : sizes[r]] for r in range(rows)], [pins[r, : sizes[r]] for r in range(rows)],
+                           list(weights), budget)
+    got = keep.cpu().numpy()
+    for r in range(rows):
+        assert np.array_equal(got[r, : sizes[r]].astype(bool), want[r]), (r, sizes[r])
+        assert (got[r, sizes[r]:] == 1).all()
+    assert (out[:, width:] == 7).all() and summary.tolist()[:4] == [budget, total, must, 0]
+
+
 def test_sum_summary_flags_a_budget_below_the_pins():
     scores = torch.ones(2, 5, dtype=torch.float64, device="cuda")
     blocks = torch.tensor([5, 5], dtype=torch.int32, device="cuda")
