@@ -214,12 +214,11 @@ int ekv_tile_shares(const float *lse, int64_t lse_plane_stride, int64_t lse_laye
 
 /*
  * ekv_tile_shares with a workspace, the same result (the same rules; float sums in another
- * fixed order): each row's layers are split over several workgroups, which write per-block
- * partial sums into the workspace, so a long row no longer sets the time on one compute unit.
- * For 4 query rows per block, rows of at most 512 blocks and at most 65536 rows, the last of a
- * row's workgroups to finish adds the partials and writes the row (it learns that it is last from
- * a per-row arrival counter in the workspace); other shapes combine them in a second kernel.
- * Replaces the same reference code as ekv_tile_shares.
+ * fixed order): each row's layers are split over several workgroups, so a long row no longer sets the time
+ * on one compute unit.  Four cells, at most 512 blocks and 65536 rows: per-block partial sums, which
+ * the row's last workgroup combines (a per-row arrival counter in the workspace).  Other shapes: two
+ * kernels that each stream the records, their peaks and totals in the workspace, or partial sums that a
+ * second kernel combines.  Replaces the same reference code as ekv_tile_shares.
  * workspace: ekv_tile_shares_workspace(nrows, width, layers) bytes of device memory (256 KB of
  * arrival counters, then the partials and their counts, which the last workgroup of a row reads
  * as they land: a slot reads zero until its value has arrived).  Fill it with zeros once before its
