@@ -929,7 +929,7 @@ struct Stat {
 };
 __device__ __forceinline__ Stat make_stat(float peak, double total) {
   const float hi = (float)total;
-  return Stat{peak, hi, (float)(total - hi)};
+  return Stat{peak, hi, hi < INFINITY ? (float)(total - hi) : 0.0f};  // past float32: no rest to an infinite total
 }
 
 // the units of a row of n blocks
@@ -1181,7 +1181,8 @@ void apply_kernel(const Params p) {
     }
     const bool has = peak != -INFINITY;
     const double inv = has ? 1.0 / total : 0.0;
-    s_stat[i] = make_float4(has ? peak : 0.0f, (float)inv, (float)(inv - (float)inv), 0.0f);
+    const float hi = (float)inv;  // infinite for a total below 2^-128: as a float32 quotient, with no rest
+    s_stat[i] = make_float4(has ? peak : 0.0f, hi, hi < INFINITY ? (float)(inv - hi) : 0.0f, 0.0f);
     contributors += has ? 1 : 0;
   }
   contributors = wave_sum_int(contributors);

@@ -307,3 +307,34 @@ def test_records_streamed_in_units_match_the_oracle(layers, rows, width, cells, 
     assert int(torch.count_nonzero(workspace)) == 0
     want = ots.normalize(ots.read_rows(planes, layers, np.arange(rows), tile), row_blocks, tile, aggregate)
     assert_close(got[0].astype(np.float64), want, 1e-6, f"{layers} x {rows} x {width} x {cells}, {aggregate}")
+
+
+@pytest.mark.parametrize("aggregate", ["mean", "max"])
+@pytest.mark.parametrize("width,cells", [(1028, 4), (516, 1), (300, 7), (520, 8)])
+def test_totals_past_float32_match_the_form_without_a_workspace(width, cells, aggregate):
+    # (layer, query row) totals above the largest float32, in a lane's sum and only across lanes, add
+    # nothing but count; totals below 2^-128 have an infinite quotient.  The stream form keeps its totals
+    # in two floats, which must not turn either into NaN.  Sums over 3 x 8 records of at most 1028 blocks
+    # in float32 on both sides: within 1e-6
+    import ekv_hip
+
+    rng = np.random.default_rng(600 + width)
+    layers, rows, tile = 3, 4, 2
+    m = rng.normal(0, 1, (layers, rows, width, cells)).astype(np.float32)
+    l = rng.uniform(0.5, 30, (layers, rows, width, cells)).astype(np.float32)
+    m[0], l[0, 0] = 0.0, 3e38
+    l[1, 1, [3, 9]] = 3e38
+    m[1, 1] = 0.0
+    m[2, 2], l[2, 2] = 0.0, 1e-42
+    dev = planes_on_device(np.stack([m, l]))
+    want = torch.empty(rows, width, device="cuda")
+    stride = rows * width * cells
+    ekv_hip.call("ekv_tile_shares", dev.data_ptr(), layers * stride, stride, width * cells, layers, cells, width, 0, 0,
+                 rows, tile, {"mean": ekv_hip.AGG_MEAN, "max": ekv_hip.AGG_MAX}[aggregate], want.data_ptr(), width,
+                 ekv_hip.stream_handle())
+    got = tile_shares.tile_shares(dev.data_ptr(), layers, layers, rows, width, cells, None, None, tile, aggregate)
+    got, want = got.cpu().numpy().astype(np.float64), want.cpu().numpy().astype(np.float64)
+    assert np.isfinite(got[[0, 1, 3]]).all() and np.isfinite(want[[0, 1, 3]]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.abs(got[ok] - want[ok]).max() <= 1e-6
