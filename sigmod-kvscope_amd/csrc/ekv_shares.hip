@@ -1420,7 +1420,8 @@ bool launch_stream(Params p, int nrows, hipStream_t s) {
   p.columns = kApplyWaves / groups;
   p.chunks = chunks_of(p.columns);
   const int64_t grid1 = team ? records * p.slices : (records + 3) / 4, grid2 = (int64_t)nrows * p.chunks;
-  if (grid1 > INT_MAX || grid2 > INT_MAX) return false;
+  // a launch has fewer than 2^32 threads
+  if (grid1 * kStreamThreads > UINT_MAX || grid2 * kApplyThreads > UINT_MAX) return false;
   const size_t lds = (size_t)p.layers * p.cells * sizeof(float4);
   auto run = [&](auto v_tag, auto c_tag) {
     constexpr int V = decltype(v_tag)::value, C = decltype(c_tag)::value;

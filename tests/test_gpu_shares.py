@@ -338,3 +338,21 @@ def test_totals_past_float32_match_the_form_without_a_workspace(width, cells, ag
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
     ok = np.isfinite(want)
     assert np.abs(got[ok] - want[ok]).max() <= 1e-6
+
+
+def test_rows_whose_streamed_launch_would_pass_the_thread_limit():
+    # 65536 rows (of one source row) x 4104 blocks x 64 cells: a workgroup per 32 blocks and row would be
+    # 8.45 million of 512 threads, past the 2^32 threads of a launch, so the layer groups' form takes
+    # the call.  Every row is the row alone, within a few float32 roundings of 64 records' mean
+    if torch.cuda.mem_get_info()[0] < 8 << 30:
+        pytest.skip("needs 8 GiB of device memory")
+    rng = np.random.default_rng(77)
+    rows, width, cells = 65536, 4104, 64
+    assert rows * -(-width * cells // 4 // 512) * 512 >= 1 << 32
+    planes = np.stack([rng.normal(0, 2, (1, 1, width, cells)), rng.uniform(1, 9, (1, 1, width, cells))])
+    dev = planes_on_device(planes.astype(np.float32))
+    ids = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    got = tile_shares.tile_shares(dev.data_ptr(), 1, 1, 1, width, cells, ids, None, 2)
+    one = tile_shares.tile_shares(dev.data_ptr(), 1, 1, 1, width, cells, ids[:1], None, 2)
+    assert torch.equal(got, got[:1].expand_as(got))
+    assert float((got[0] - one[0]).abs().max()) <= 1e-8
