@@ -415,10 +415,17 @@ inline int pass_grid(int rows, int width, int cus) {
   return std::min((rows + side - 1) / side, cus);
 }
 
-// Workgroup w's region of the list: an equal share of the list's kCandPerRow pairs a row.
+// Workgroup w's region of the list: kCandPerRow pairs for each row that its workers take (the first
+// rows % workers workers take one more than the others), so a list overflows by its own rows' blocks
+// whatever the others have: an equal share of the room overflowed at 300 x 4096 blocks of Dirichlet(0.3)
+// shares, where 44 workgroups have two rows, and the call took 63 us (55 with this).
+template <int SPAN>
 __device__ __forceinline__ void cand_region(int rows, int w, int grid, long long &first, int &room) {
-  room = (int)((long long)kCandPerRow * rows / grid);
-  first = (long long)room * w;
+  constexpr int kSide = PassRows<SPAN>::kSide;
+  const int workers = grid * kSide, per = rows / workers, extra = rows - per * workers;
+  auto rows_before = [&](int worker) { return (long long)per * worker + min(worker, extra); };
+  first = kCandPerRow * rows_before(w * kSide);
+  room = (int)(kCandPerRow * rows_before((w + 1) * kSide) - first);
 }
 
 constexpr int kHistRows = 2;  // rows whose blocks a pass's workgroup loads together
@@ -436,7 +443,7 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const Params p, int 
   __syncthreads();
   long long region;
   int room;
-  cand_region(p.rows, blockIdx.x, gridDim.x, region, room);
+  cand_region<SPAN>(p.rows, blockIdx.x, gridDim.x, region, room);
   const unsigned int digit_mask = (1u << bits) - 1u;
   const unsigned long long prefix = s->prefix, mask = s->mask, threshold = s->threshold;
   const int lane = lane_id();
@@ -572,7 +579,7 @@ __global__ __launch_bounds__(kHistThreads) void sum_keep_kernel(const Params p) 
   };
   long long region;
   int room;
-  cand_region(p.rows, blockIdx.x, gridDim.x, region, room);
+  cand_region<SPAN>(p.rows, blockIdx.x, gridDim.x, region, room);
   const bool second_ran = mode == kSelect && !error && !s->done_first;
   const unsigned int listed = second_ran ? p.cand_count[blockIdx.x] : 0u;
   if (second_ran && listed <= (unsigned int)room) {

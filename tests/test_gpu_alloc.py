@@ -217,6 +217,32 @@ def test_sum_rows_side_by_side(rows, width, kind):
     assert (out[:, width:] == 7).all() and summary.tolist()[:4] == [budget, total, must, 0]
 
 
+@pytest.mark.parametrize("rows_past,per_cu,width", [(44, 1, 3000), (1, 1, 2049), (100, 4, 1500)])
+def test_sum_lists_have_room_for_every_row_of_their_workgroup(rows_past, per_cu, width):
+    # row counts that leave some workgroups of the passes a row more than the others (one or four rows side
+    # by side): 900 blocks a row in one first digit are within the 1024 pairs that a row brings to its
+    # workgroup's list, so every one of them is found in the workspace (a list without room for a
+    # workgroup's second row makes each later pass read the rows again)
+    rows = torch.cuda.get_device_properties(0).multi_processor_count * per_cu + rows_past
+    rng = np.random.default_rng(rows + width)
+    scores = np.zeros((rows, width))
+    for r in range(rows):
+        listed = rng.choice(np.arange(1, width - 1), size=900, replace=False)
+        scores[r, listed] = rng.uniform(1.0, 1.5, size=900)  # shares of 900 such: within a quarter of 1 / 1125
+    need = allocation.sum_workspace_bytes(rows)
+    workspace = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    budget = 2 * rows + 450 * rows
+    keep, summary = allocation.sum_keep(
+        torch.from_numpy(scores).cuda(), torch.full((rows,), width, dtype=torch.int32, device="cuda"), budget=budget,
+        workspace=workspace)
+    assert summary.tolist()[:4] == [budget, rows * width, 2 * rows, 0] and int(keep.sum()) == budget
+    words = workspace[(-workspace.data_ptr()) % 8:]
+    words = words[: words.numel() // 8 * 8].view(torch.int64).cpu().numpy()
+    row, block = np.nonzero(scores)
+    tie_keys = (block.astype(np.int64) << 16) | (65535 - row)
+    assert np.isin(tie_keys, words).all()
+
+
 def test_sum_summary_flags_a_budget_below_the_pins():
     scores = torch.ones(2, 5, dtype=torch.float64, device="cuda")
     blocks = torch.tensor([5, 5], dtype=torch.int32, device="cuda")
