@@ -405,10 +405,13 @@ struct PassRows {
 // The threads of a row, and the passes' workgroups.  An eighth of the width covers a row, but fewer than
 // ~32 workgroups lose more than they save: calls of 911 x 299 blocks take 67 us at 64 threads a row (90 at
 // 1024), 323 x 247 76 at 256 (93 at 1024), 128 x 512 with masks 50 at 256, 54 at 64 (8 workgroups) and 51 at
-// 1024, 14 x 1979 39 at 1024 and 42 at 256.
+// 1024, 14 x 1979 39 at 1024 and 42 at 256.  Rows of more than 1024 blocks can also outgrow their list, and
+// then the later passes read them again, on as few workgroups: 200 x 2048 with 70% zero shares takes 117 us
+// at 256 threads and 101 at 1024, 256 x 1600 78 and 102, 400 x 2048 118 and 110, 900 x 2048 125 and 151.
 inline int pass_span(int rows, int width) {
   if (width <= 64 * kRun && rows >= 512) return 64;
-  return width <= 256 * kRun && rows >= 128 ? 256 : kHistThreads;
+  const int from = width <= kCandPerRow ? 128 : width <= 1792 ? 256 : 600;
+  return width <= 256 * kRun && rows >= from ? 256 : kHistThreads;
 }
 inline int pass_grid(int rows, int width, int cus) {
   const int side = kHistThreads / pass_span(rows, width);

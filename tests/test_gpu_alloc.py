@@ -189,7 +189,8 @@ def test_maxmin_more_than_65536_requests():
 
 
 @pytest.mark.parametrize("rows,width", [(127, 300), (128, 512), (129, 513), (130, 2048), (131, 2049), (511, 40),
-                                        (512, 512), (513, 511), (700, 513), (1025, 64)])
+                                        (512, 512), (513, 511), (700, 513), (1025, 64), (128, 1025), (255, 1300),
+                                        (256, 1792), (300, 1793), (600, 2048)])
 @pytest.mark.parametrize("kind", ["shares", "ties"])
 def test_sum_rows_side_by_side(rows, width, kind):
     # the passes take a row with 64, 256 or 1024 threads by the number of rows and the width: both sides of
