@@ -558,3 +558,58 @@ def test_maxmin_many_requests(rows):
         budget = max(int(frac * total), must)
         reqs = [allocation.Request(scores=s, pinned=p) for s, p in zip(scores, pinned)]
         assert same(allocation.allocate(reqs, budget, "maxmin"), oa.allocate_maxmin(scores, pinned, budget)), frac
+
+
+def maxmin_order_and_totals(scores, pins, width, masked):
+    """A call's requests' open blocks in sorted order and their running totals, read from the workspace
+    (rows of at most 12288 blocks), beside NumPy's; the keep is checked against the oracle."""
+    rows, lengths = len(scores), [len(x) for x in scores]
+    grid, mask = np.zeros((rows, width)), np.zeros((rows, width), np.uint8)
+    for r in range(rows):
+        grid[r, : lengths[r]], mask[r, : lengths[r]] = scores[r], pins[r]
+    need = allocation.maxmin_workspace_bytes(rows, width)
+    workspace = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    must = sum(int(p.sum()) for p in pins)
+    budget = must + (sum(lengths) - must) // 2
+    keep, summary = allocation.maxmin_keep(
+        torch.from_numpy(grid).cuda(), torch.tensor(lengths, dtype=torch.int32, device="cuda"), budget=budget,
+        pinned=torch.from_numpy(mask).cuda() if masked else None, workspace=workspace)
+    assert summary.tolist()[:4] == [budget, sum(lengths), must, 0]
+    want_keep, keep = oa.allocate_maxmin(scores, pins, budget), keep.cpu().numpy().astype(bool)
+    raw = workspace.cpu().numpy()
+    prefix = (-workspace.data_ptr()) % 256 + need - 256 - (rows * width * 8 + 255) // 256 * 256
+    vals = prefix - (rows * width * 4 + 255) // 256 * 256
+    for r in range(rows):
+        share = oa.shares(scores[r])
+        blocks = np.flatnonzero(~pins[r])
+        blocks = blocks[np.argsort(-share[blocks], kind="stable")]
+        totals = np.cumsum(share[blocks])
+        got_order = raw[vals + r * width * 4: vals + (r * width + len(blocks)) * 4].view(np.int32)
+        got = raw[prefix + r * width * 8: prefix + (r * width + len(blocks)) * 8].view(np.float64)
+        assert np.array_equal(got_order, blocks), (r, lengths[r], int(np.argmax(got_order != blocks)))
+        assert got.tobytes() == totals.tobytes(), (r, lengths[r], int(np.argmax(got != totals)))
+        assert np.array_equal(keep[r, : lengths[r]], want_keep[r]), (r, lengths[r])
+
+
+def share_keys(scores, pins):
+    """The order-preserving keys of a request's open shares (not negative): larger share, larger key."""
+    share = oa.shares(scores)[~pins]
+    return share.view(np.uint64) | np.uint64(1 << 63)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("kind", [2.0 ** -40, 2.0 ** -30, 2.0 ** -26, "ties"])
+def test_maxmin_rows_past_8192_blocks_sorted_again(kind, masked):
+    # a call with rows of 8193 to 12288 blocks takes the LDS radix sort for every request, with 1, 2, 4, 8 or
+    # 12 keys a thread; shares that agree in their top 40 bits out of order below are sorted again
+    # (spreads of a few float64 ulps), equal ones keep block order
+    rng = np.random.default_rng(42 if kind == "ties" else int(-np.log2(kind)))
+    scores, pins = [], []
+    for n in (12288, 9000, 8193, 8192, 5000, 4096, 2049, 2048, 1025, 1024, 700, 64):
+        scores.append(np.round(rng.random(n) * 8) / 8 if kind == "ties" else 0.5 * (1.0 + rng.integers(0, 7, n) * kind))
+        pins.append(oa.default_pins(n) if not masked else rng.random(n) < 0.05)
+        top, low = share_keys(scores[-1], pins[-1]) >> 24, share_keys(scores[-1], pins[-1]) & 0xffffff
+        order = np.argsort(top, kind="stable")[::-1]  # runs of equal top bits, each from its last block
+        again = (top[order][1:] == top[order][:-1]) & (low[order][1:] < low[order][:-1])
+        assert again.any() == (kind != "ties" and kind < 2.0 ** -28), n
+    maxmin_order_and_totals(scores, pins, 12288, masked)
