@@ -613,3 +613,111 @@ def test_maxmin_rows_past_8192_blocks_sorted_again(kind, masked):
         again = (top[order][1:] == top[order][:-1]) & (low[order][1:] < low[order][:-1])
         assert again.any() == (kind != "ties" and kind < 2.0 ** -28), n
     maxmin_order_and_totals(scores, pins, 12288, masked)
+
+
+def bucket_case(scores, pins):
+    """How the row kernel's ranks take a request: the bits that every bucket has to fix (2 and more: the
+    shares span more than 512 binades and take the radix sort)."""
+    keys = share_keys(scores, pins)
+    keys = keys[keys > np.uint64(1 << 63)]
+    span = int(keys.max() - keys.min())
+    cut = max(0, (span | 1).bit_length() - 9)
+    cut += (span >> cut) >= 511
+    return max(0, cut + 13 - 64)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("width", [512, 1024, 4096, 8192])
+def test_maxmin_shares_over_many_binades(width, masked):
+    # shares over 200 to 600 binades: below 256 a bucket's word holds all that the bucket leaves open;
+    # from there to 511 every bucket has to fix one bit more; past that the request takes the radix
+    # sort.  Whole rows with several blocks a coarse bin, the order read from the workspace (the totals
+    # stop changing after the first binades)
+    rng = np.random.default_rng(width + masked)
+    scores, pins, cases = [], [], []
+    for binades in (200, 254, 258, 300, 400, 500, 508, 513, 600):
+        x = np.ldexp(1.0 + rng.random(width), rng.integers(-binades, 1, width))
+        x[[width // 3, width // 2]] = [1.0, np.ldexp(1.0, -binades)]  # the whole range, unpinned
+        pin = rng.random(width) < 0.05 if masked else oa.default_pins(width)
+        pin[[width // 3, width // 2]] = False
+        scores.append(x)
+        pins.append(pin)
+        cases.append(bucket_case(x, pin))
+    assert cases == [0, 0, 1, 1, 1, 1, 1, 2, 2]
+    maxmin_order_and_totals(scores, pins, width, masked)
+
+
+def window_ties(share, threads):
+    """The scan windows of a request's sorted open shares, as the row kernel takes them with this many
+    threads: (ties in the window, whether it is a wide one) for each."""
+    totals = np.cumsum(share)
+    windows, pos, n = [], 0, len(share)
+    alone, wide = True, False
+    t = -0.0
+    while pos < n:
+        if alone or not t > 0.0:
+            pos = min(pos + 64, n)
+            t, alone = totals[pos - 1], False
+            continue
+        u = np.spacing(t)
+        asked = min(n - pos, (8 if wide else 2) * threads)
+        y = share[pos: pos + asked] / u  # exact: u is a power of two
+        tie = y - np.floor(y) == 0.5
+        before = np.concatenate([[t], totals[pos: pos + asked - 1]])
+        under = y < 2.0 ** 53 - before / u
+        windows.append((int(tie.sum()), wide))
+        if tie.sum() > 64:
+            asked = min(n - pos, 2 * threads)
+            stop = ~under[:asked] | tie[:asked]
+            taken = int(np.argmax(stop)) if stop.any() else asked
+            alone = taken < asked
+        else:
+            taken = int(np.argmax(~under)) if not under.all() else asked
+            alone, wide = taken < 64, taken == asked
+        if taken:
+            t = totals[pos + taken - 1]
+        pos += taken
+        if pos < n and taken < asked and not alone:
+            t = totals[pos]
+            pos += 1
+    return windows
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("width,threads", [(512, 256), (1024, 256), (4096, 512), (8192, 512)])
+def test_maxmin_totals_with_many_ties_in_a_window(width, threads, masked):
+    # a tie (a share that is an odd multiple of half the total's last bit) is resolved in place up to 64 a
+    # window; more of them end the window at the first.  Shares in units of 2^-54 on a total in [1/2, 1),
+    # whose last bit is 2^-53: odd ones tie.  The first and last block, pinned, hold the rest of the
+    # request, set so that NumPy's total is 1 and the shares are the scores.
+    scores, pins, seen = [], [], []
+
+    def row(big, small):
+        x = np.concatenate([[0.0, big], np.asarray(small, float) * 2.0 ** -54, [0.25]])
+        x[0] = 0.75 - big - np.sum(x[2:-1])
+        while np.sum(x) != 1.0:
+            x[0] += 1.0 - np.sum(x)
+        pin = np.zeros(len(x), bool)
+        pin[[0, -1]] = True
+        scores.append(x)
+        pins.append(pin)
+        assert np.array_equal(oa.shares(x), x)
+        seen.append(window_ties(np.sort(x[1:-1])[::-1], threads))
+
+    rng = np.random.default_rng(width + masked)
+    m = width - 3  # small shares of a whole row
+    row(0.6, np.full(m, 3))  # every value ties
+    row(0.6, rng.choice([2, 3, 4, 5, 6, 7], m))
+    for count in (64, 65):  # that many ties in the first window
+        row(0.6, np.concatenate([np.full(100, 4), np.full(count, 3), np.full(m - 100 - count, 2)]))
+        assert seen[-1][0] == (count, False)
+    if width > 3 * threads:  # a whole window without ties, then a wide one with many, 64 and 65
+        first = 64 + 2 * threads
+        for count in (64, 65, m - first):
+            row(0.6, np.concatenate([np.full(first, 4), np.full(count, 3), np.full(m - first - count, 2)]))
+            assert any(w and (ties == count or 65 < ties < count) for ties, w in seen[-1])
+    row(0.5 - 3 * 150 * 2.0 ** -54, np.full(m, 3))  # the total enters [1/2, 1) after 150 of them
+    row(0.6, np.full(m // 2, 7))
+    assert any(ties > 64 for ties, _ in seen[0]) and any(ties > 64 for ties, _ in seen[1])
+    assert any(ties > 64 for ties, _ in seen[-2])
+    maxmin_order_and_totals(scores, pins, width, masked)
