@@ -224,9 +224,11 @@ __global__ __launch_bounds__(kPrepThreads) void prepare_kernel(const Params p) {
 // the requests' pinned, existing and open blocks, summed over the rows' statistics by one
 // workgroup, then the budget's mode (allocation.py:57-76) and the select's start; the state
 // (histogram, flags, counters) is cleared first
-// COHERENT: the statistics were stored by this launch's other workgroups (store_row_stat).
+// COHERENT: the statistics were stored by this launch's other workgroups (store_row_stat).  Inlined: as a call
+// it cost its kernel registers and scratch throughout (mm_rows_kernel<512, 8> 94 VGPRs, 74 without;
+// 4096 x 4096 blocks 405 us, 284).
 template <int NT, bool COHERENT = false>
-__device__ void decide(const Params &p) {
+__device__ __forceinline__ void decide(const Params &p) {
   __shared__ long long s_red[3][NT / kWave];
   {
     unsigned long long *w = (unsigned long long *)p.state;
@@ -1500,23 +1502,26 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
 // radix sort), so those and the block's 13-bit index are one 64-bit word, and every comparison is of the
 // whole key and then the index: the order is the stable one whatever order the buckets were filled in.
 // Bucket bounds come from a bitmap of the buckets' first positions: a wave ranks 64 consecutive positions
-// and reads one word of it.  A request with a bucket of more than kBucketLimit blocks (many equal
-// shares, or shares that crowd together far below the bins' width) or a NaN share takes the radix sort
-// instead.
+// and reads one word of it.  Buckets of more than kEqualFrom equal shares are put in block order without
+// comparing (order_equal).  A request with a bucket of more than kBucketLimit blocks that are not all
+// equal (shares that crowd together far below the bins' width) or with NaN among other shares takes the
+// radix sort instead, on half the threads that mm_sort_kernel has: 1024 x U[1, 8192] 340 us, 316 there.
 //
 // The running totals are scan_chunk's exact windows over the whole workgroup, in which only a new binade
 // ends a window (scan_window), so a long request takes ~5 windows.
 //
-// At 1024 x U[1, 8192]: 115 us, where the totals, the radix sort of every request and a scan wave and a
-// level wave a request took 12 + 99 + 55; at 128 x U[32, 512]: 17 us for 6 + 12 + 25.  Bound by a
+// At 1024 x U[1, 8192]: 87 us, where the totals, the radix sort of every request and a scan wave and a
+// level wave a request took 12 + 99 + 55; at 128 x U[32, 512]: 18 us for 6 + 12 + 25.  Bound by a
 // request's chain of phases, each a few LDS round trips and dependent float64 operations between
-// barriers (~120000 cycles for 8192 blocks: loads 15, total 7, keys 7, ranks 45, totals 25, levels 7),
+// barriers (~120000 cycles for 8192 blocks while it took 115 us: loads 15, total 7, keys 7, ranks 45, totals
+// 25, levels 7),
 // two 8-wave workgroups a CU (80 KB of LDS each) filling each other's gaps.  1024 threads a request at 64
 // VGPRs spilled (328 us); __syncthreads' waits for global stores cost ~5 us a request.
 constexpr int kRowsWidth = 8 * kSortThreads;  // the widest request
 static_assert(kRowsWidth <= 1 << 13, "a block index fits a bucket sort's word");
 constexpr int kCoarse = 512;                  // coarse bins
 constexpr int kBucketLimit = 128;
+constexpr int kEqualFrom = 64;                // larger buckets are looked at for one key (order_equal)
 constexpr int kTies = 64;  // ties of a scan window resolved in place
 constexpr int kRowIndexBits = 13;             // block indices in a bucket sort's words
 
@@ -1554,7 +1559,8 @@ struct RowLds {
     int pin_count[NT / kWave * ITEMS];
   };
   double base;
-  int flag, stop, ties, tie[kTies];
+  int flag, stop, ties;
+  int tie[kRowsWidth / kEqualFrom];  // scan_window's ties; order_equal's buckets
   unsigned short zero_count[NT / kWave * ITEMS];
 };
 
@@ -1592,25 +1598,86 @@ __device__ __forceinline__ void block_max2_u64(unsigned long long &a, unsigned l
   lds_barrier();
 }
 
+// Buckets of more than kEqualFrom blocks (lds.tie, by first position / kEqualFrom: first position <<
+// kIndexBits | blocks), a wave a bucket: the words of one key's are put in block order, from a bitmap of
+// the blocks in the buckets' words, which are free by now.  One of more keys is taken off the list, or
+// lds.flag set where it is over the limit.  Calls of 64 x U[4096, 8192] blocks with 65 values 123 us, 153
+// by the radix sort for buckets over the limit; 2172 x 3188 equal shares 349, 465; 1024 x U[1, 8192] of nine
+// values 219, 269.
+template <int NT, int MAX_ITEMS>
+__device__ __forceinline__ void order_equal(int positive, RowLds<NT, MAX_ITEMS> &lds) {
+  constexpr int kWords = RowLds<NT, MAX_ITEMS>::kCap / 32;
+  static_assert(NT / kWave * kWords <= RowLds<NT, MAX_ITEMS>::kBuckets / 2, "a bitmap a wave");
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(phase_thread() / kWave);
+  unsigned int *bits = lds.bucket + wave * kWords;
+#pragma unroll 1
+  for (int j = wave; j * kEqualFrom < positive; j += NT / kWave) {
+    const int tie = __builtin_amdgcn_readfirstlane(lds.tie[j]);
+    if (tie == 0) continue;
+    const int first = tie >> kIndexBits, count = tie & ((1 << kIndexBits) - 1);
+    const unsigned long long key = lds.elem[first] >> kRowIndexBits;
+    uint64_t other = __ballot((lds.elem[first + lane] >> kRowIndexBits) != key);  // most show it here
+    if (other == 0ull) {
+      for (int w = lane; w < kWords; w += kWave) bits[w] = 0u;
+      __builtin_amdgcn_wave_barrier();
+      bool mine = false;
+      // a lane takes an odd number of neighbours, the lanes' blocks then seldom share a word or a bank
+      const int run = ((count + kWave - 1) / kWave) | 1, to = min(count, (lane + 1) * run);
+#pragma unroll 1
+      for (int q = lane * run; q < to; ++q) {
+        const unsigned long long e = lds.elem[first + q];
+        const int b = (int)(e & ((1ull << kRowIndexBits) - 1ull));
+        mine |= (e >> kRowIndexBits) != key;
+        atomicOr(&bits[b >> 5], 1u << (b & 31));
+      }
+      __builtin_amdgcn_wave_barrier();
+      other = __ballot(mine);
+    }
+    if (other != 0ull) {
+      lds.tie[j] = 0;
+      if (count > kBucketLimit) lds.flag = 1;
+      continue;
+    }
+    int before = first;
+#pragma unroll 1
+    for (int w0 = 0; w0 < kWords; w0 += kWave) {
+      const unsigned int word = w0 + lane < kWords ? bits[w0 + lane] : 0u;
+      const int inc = wave_inclusive_scan(__popc(word));
+      const int at = before + inc - __popc(word), turn = lane & 31;
+      // a lane starts at a bit of its own: whole words would all store to one bank
+      for (unsigned int left = __builtin_rotateright32(word, turn); left != 0u; left &= left - 1u) {
+        const int bit = (__ffs((int)left) - 1 + turn) & 31;
+        lds.elem[at + __popc(word & ((1u << bit) - 1u))] =
+            (key << kRowIndexBits) | (unsigned long long)(32 * (w0 + lane) + bit);
+      }
+      before += __builtin_amdgcn_readlane(inc, kWave - 1);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // The exact ranks of a request's open blocks: pos_of[b] in LDS for each, and vals_out.  k: the thread's
 // keys, of blocks i * NT + thread (0: pinned or past the row).  False, with nothing done, when a bucket
-// is over the limit.
+// over the limit holds two keys, or some of the shares are NaN.
 template <int NT, int ITEMS, int MAX_ITEMS>
 __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS], int open, int32_t *vals,
                                              RowLds<NT, MAX_ITEMS> &lds) {
   constexpr unsigned long long kZero = 1ull << 63;  // the key of a zero share; positive shares' are above it
+  constexpr unsigned long long kNan = 1ull;
   const int lane = lane_id();
   int tid = phase_thread();
   unsigned long long top = 0ull, under = 0ull;  // the largest key, and the largest complement of one
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
-    if (k[i] > kZero) {
-      top = k[i] > top ? k[i] : top;
-      under = ~k[i] > under ? ~k[i] : under;
-    }
+    if (k[i] > kZero) top = k[i] > top ? k[i] : top;
+    if (k[i] > kZero || k[i] == kNan) under = ~k[i] > under ? ~k[i] : under;
   }
   block_max2_u64<NT>(top, under, lds.scan64);
   const unsigned long long bottom = ~under;
+  const bool nan = bottom == kNan;
+  if (nan && top != 0ull) return false;
+  const unsigned long long last = nan ? kNan : kZero;  // a request of NaN shares only is in block order
   const unsigned long long span = top > bottom ? top - bottom : 0ull;
   // coarse bin of x: x >> cut, at most kCoarse - 2
   int cut = max(0, 64 - (int)__builtin_clzll(span | 1ull) - 9);
@@ -1620,16 +1687,16 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
   for (int j = tid; j < kCoarse; j += NT) lds.coarse[j] = 0u;
   for (int j = tid; j < lds.kBuckets / 2; j += NT) lds.bucket[j] = 0u;
   for (int j = tid; j < (int)(sizeof(lds.heads) / 4); j += NT) lds.heads[j] = 0u;
-  if (tid == 0) lds.flag = 0;
+  for (int j = tid; j < kRowsWidth / kEqualFrom; j += NT) lds.tie[j] = 0;
+  if (tid == 0) lds.flag = lds.ties = 0;
   lds_barrier();
   tid = phase_thread();
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i)
   {
     if (k[i] > kZero) atomicAdd(&lds.coarse[(int)((top - k[i]) >> cut)], 1u);
-    const uint64_t zeros = __ballot(k[i] == kZero);
+    const uint64_t zeros = __ballot(k[i] == last);
     if (lane == 0) lds.zero_count[i * (NT / kWave) + (tid / kWave)] = (unsigned short)__popcll(zeros);
-    if (k[i] == 1ull) lds.flag = 1;  // NaN
   }
   lds_barrier();
   tid = phase_thread();
@@ -1704,7 +1771,6 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
       mine += a + b;
       most = max(most, max(a, b));
     }
-    if (most > kBucketLimit) lds.flag = 1;
     int all;
     int at = block_exclusive_scan<NT, true>(mine, lds.scan, all);
 #pragma unroll
@@ -1712,6 +1778,11 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
       const int j = tid * kPer + q;
       const int a = (int)(w[q] & 0xffffu), b = (int)(w[q] >> 16);
       if (j < kWords) lds.bucket[j] = (unsigned int)at | ((unsigned int)(at + a) << 16);
+      if (most > kEqualFrom) {  // their positions are so far apart that each has an entry of its own
+        lds.ties = 1;
+        if (a > kEqualFrom) lds.tie[at / kEqualFrom] = (at << kIndexBits) | a;
+        if (b > kEqualFrom) lds.tie[(at + a) / kEqualFrom] = ((at + a) << kIndexBits) | b;
+      }
       if (a > 0) atomicOr(&lds.heads[at >> 5], 1u << (at & 31));
       if (b > 0) atomicOr(&lds.heads[(at + a) >> 5], 1u << ((at + a) & 31));
       at += a + b;
@@ -1719,7 +1790,8 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
   }
   lds_barrier();
   tid = phase_thread();
-  if (lds.flag != 0) return false;
+  const int positive = open - lds.stop;  // the zero shares follow in block order
+  if (nan && positive != 0) return false;
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
     if (i % 4 == 0) keep_order();
@@ -1731,9 +1803,16 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
     }
   }
   lds_barrier();
+  if (lds.ties != 0) {
+    order_equal<NT, MAX_ITEMS>(positive, lds);
+    lds_barrier();
+    if (lds.flag != 0) return false;
+  }
   tid = phase_thread();
-  const int positive = open - lds.stop;  // the zero shares follow in block order
   // positions i * NT + thread: the bucket's bounds from the bitmap, then the blocks of it before this one
+  // (none are counted where order_equal has put them in their places; the bounds of a bucket over the limit come
+  // out further apart than the limit, but no word of the bitmap past that is read)
+  constexpr int kLimitWords = kBucketLimit / 32;
   uint32_t moved[ITEMS];  // rank | index << 16
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i) {
@@ -1748,21 +1827,24 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
         from = p0 + 63 - __clzll((long long)upto);
       } else {  // the bucket starts in an earlier word (position 0 is a head)
         int w = w0 - 1;
-        while (w > 0 && lds.heads[w] == 0u) --w;
+        while (w > max(0, w0 - kLimitWords) && lds.heads[w] == 0u) --w;
         from = 32 * w + 31 - __clz((int)lds.heads[w]);
       }
       if (after != 0ull) {
         to = p0 + __ffsll((long long)after) - 1;
       } else {
         int w = w0 + 2;
-        while (32 * w < positive && lds.heads[w] == 0u) ++w;
-        to = 32 * w < positive ? 32 * w + __ffs((int)lds.heads[w]) - 1 : positive;
+        while (32 * w < positive && w < w0 + 2 + kLimitWords && lds.heads[w] == 0u) ++w;
+        to = 32 * w;
+        if (to < positive && w < w0 + 2 + kLimitWords) to += __ffs((int)lds.heads[w]) - 1;
       }
       to = min(to, positive);
       if (p < positive) {
         const unsigned long long e = lds.elem[p];
         int rank = from;
-        if (to - from > 1) {
+        if (to - from > kBucketLimit || (to - from > kEqualFrom && lds.tie[from / kEqualFrom] != 0)) {
+          rank = p;
+        } else if (to - from > 1) {
           for (int q = from; q < to; q += 4) {  // four reads in flight
             unsigned long long x[4];
 #pragma unroll
@@ -1785,8 +1867,8 @@ __device__ __forceinline__ bool bucket_ranks(const unsigned long long (&k)[ITEMS
       vals[rank] = b;
       lds.pos_of[b] = (unsigned short)rank;
     }
-    const uint64_t zeros = __ballot(k[i] == kZero);
-    if (k[i] == kZero) {
+    const uint64_t zeros = __ballot(k[i] == last);
+    if (k[i] == last) {
       const int rank = positive + lds.zero_count[i * (NT / kWave) + tid / kWave] +
                        __builtin_amdgcn_mbcnt_hi((uint32_t)(zeros >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)zeros, 0u));
       vals[rank] = i * NT + tid;

@@ -721,3 +721,59 @@ def test_maxmin_totals_with_many_ties_in_a_window(width, threads, masked):
     assert any(ties > 64 for ties, _ in seen[0]) and any(ties > 64 for ties, _ in seen[1])
     assert any(ties > 64 for ties, _ in seen[-2])
     maxmin_order_and_totals(scores, pins, width, masked)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("width", [512, 1024, 4096, 8192])
+def test_maxmin_equal_shares_keep_block_order(width, masked):
+    # more than 64 blocks in one of the ranks' buckets: of one share they are put in block order from a
+    # bitmap; up to 128 of several shares are ranked by comparing, more send the request to the radix
+    # sort.  Group sizes around both limits, one group, as many groups as fit (short and whole rows), in
+    # random block order; the order read from the workspace
+    rng = np.random.default_rng(width + masked)
+    scores, pins = [], []
+
+    def row(values):
+        x = rng.permutation(np.asarray(values, float))
+        scores.append(x)
+        pin = rng.random(len(x)) < 0.03 if masked else oa.default_pins(len(x))
+        if masked and len(x) < width:
+            pin[:] = False  # the groups whole, and no pins at all
+        pins.append(pin)
+
+    for n in sorted({width, width - 1, width // 2 + 1}):
+        row(np.full(n, 0.3))
+        for size in (63, 64, 65, 66, 128, 129, 130, 131, 300):
+            row(1.0 + np.arange(n) // size)
+            row(np.where(np.arange(n) % 3, 2.0 ** -(1.0 + np.arange(n) // size % 40), 0.0))
+    # one far share widens the bins, so that neighbouring float64 values share a bucket
+    for size in (60, 64, 65, 100, 128, 129, 200):
+        crowd = 1.0 + rng.integers(0, 3, size) * 2.0 ** -52
+        row(np.concatenate([crowd, [1e-30, 1e-30], np.full(min(width - size - 2, 150), 2.0)]))
+    row(np.concatenate([np.full(64, 1.0), [1.0 + 2.0 ** -52], [1e-30, 1e-30]]))
+    row(np.concatenate([np.full(200, 1.0), [1.0 + 2.0 ** -52], [1e-30, 1e-30]]))
+    maxmin_order_and_totals(scores, pins, width, masked)
+
+
+@pytest.mark.parametrize("width", [512, 1024, 4096, 8192])
+def test_maxmin_nan_shares_keep_block_order(width):
+    # a NaN score makes every share of its request NaN: equal, in block order.  An infinite one leaves
+    # zeros, which come before the NaN share of its own block
+    rows, far = 4, 5
+    grid = np.random.default_rng(width).random((rows, width))
+    lengths = [width, width - 1, 3, width]
+    grid[:3, 1] = np.nan
+    grid[3, far] = np.inf
+    need = allocation.maxmin_workspace_bytes(rows, width)
+    workspace = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    allocation.maxmin_keep(torch.from_numpy(grid).cuda(), torch.tensor(lengths, dtype=torch.int32, device="cuda"),
+                           budget=sum(lengths) // 2, workspace=workspace)
+    raw = workspace.cpu().numpy()
+    vals = (-workspace.data_ptr()) % 256 + need - 256 - (rows * width * 8 + 255) // 256 * 256 \
+        - (rows * width * 4 + 255) // 256 * 256
+    for r, n in enumerate(lengths):
+        want = np.arange(1, n - 1)
+        if r == 3:
+            want = np.concatenate([want[want != far], [far]])
+        got = raw[vals + r * width * 4: vals + (r * width + n - 2) * 4].view(np.int32)
+        assert np.array_equal(got, want), r
