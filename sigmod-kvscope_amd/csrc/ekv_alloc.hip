@@ -408,11 +408,13 @@ struct PassRows {
 // ~32 workgroups lose more than they save: calls of 911 x 299 blocks take 67 us at 64 threads a row (90 at
 // 1024), 323 x 247 76 at 256 (93 at 1024), 128 x 512 with masks 50 at 256, 54 at 64 (8 workgroups) and 51 at
 // 1024, 14 x 1979 39 at 1024 and 42 at 256.  Rows of more than 1024 blocks can also outgrow their list, and
-// then the later passes read them again, on as few workgroups: 200 x 2048 with 70% zero shares takes 117 us
-// at 256 threads and 101 at 1024, 256 x 1600 78 and 102, 400 x 2048 118 and 110, 900 x 2048 125 and 151.
+// then the later passes read them again, on as few workgroups, so the line rises with the width (256 threads
+// and 1024, whole rows): 130 x 1750 of Dirichlet(0.1) shares 53.1 us and 51.9, of crowded ones 62.9 and 57.1;
+// 200 x 1280 51.6 and 54.8, 66.6 and 68.4; 200 x 2000 54.9 and 56.1, 73.1 and 70.6; 260 x 2048 55.9 and 59.4,
+// 64.7 and 66.1.  Past the line the most lost: 250 x U[125, 2000], 70% zero shares, 111 and 104.
 inline int pass_span(int rows, int width) {
   if (width <= 64 * kRun && rows >= 512) return 64;
-  const int from = width <= kCandPerRow ? 128 : width <= 1792 ? 256 : 600;
+  const int from = width <= 1280 ? 128 : width <= 1536 ? 192 : 256;
   return width <= 256 * kRun && rows >= from ? 256 : kHistThreads;
 }
 inline int pass_grid(int rows, int width, int cus) {
