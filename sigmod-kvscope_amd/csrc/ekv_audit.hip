@@ -22,6 +22,7 @@
 //    each lane's slice with the query slice (v_dot2 / FMA) and reduces over the lanes of a row.
 //  * Timer.  With a cycles buffer each wave adds its s_memtime durations to cycles[row] with a
 //    vector 64-bit atomic (the pass's per-row timer, mlir_pass/lib/eKVTimer.cpp:1348-1387).
+#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -1281,20 +1282,22 @@ constexpr int kStageThreads = 256;  // at most; a row of fewer pieces takes as m
 
 __global__ __launch_bounds__(kStageThreads) void stage_queries_kernel(
     const char *q, int64_t q_stride_token, int64_t q_stride_head, int32_t head_first, int32_t heads,
-    int32_t row_bytes, const int32_t *qrow, const uint8_t *select, const uint32_t *flag, char *staged,
+    int32_t row_bytes, const int32_t *qrow, const uint8_t *select, const uint32_t *flag, int32_t rows, char *staged,
     int64_t staged_row_stride) {
-  const int r = blockIdx.x;
   const unsigned pieces_head = (unsigned)row_bytes / 16;
   const uint32_t on = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint8_t chosen = select[r];
-  const int token = qrow[r];
-  if (on == 0u || chosen == 0) return;
-  for (unsigned i = blockIdx.y * blockDim.x + threadIdx.x; i < (unsigned)heads * pieces_head;
-       i += gridDim.y * blockDim.x) {
-    const unsigned h = i / pieces_head, pc = i - h * pieces_head;
-    const u32x4 v = *(const u32x4 *)(q + (int64_t)token * q_stride_token +
-                                     (int64_t)(head_first + (int)h) * q_stride_head + 16 * pc);
-    *(u32x4 *)(staged + (int64_t)r * staged_row_stride + 16 * (int64_t)i) = v;
+  for (unsigned r = blockIdx.x; r < (unsigned)rows; r += gridDim.x) {
+    const uint8_t chosen = select[r];
+    const int token = qrow[r];
+    if (on == 0u) return;
+    if (chosen == 0) continue;
+    for (unsigned i = blockIdx.y * blockDim.x + threadIdx.x; i < (unsigned)heads * pieces_head;
+         i += gridDim.y * blockDim.x) {
+      const unsigned h = i / pieces_head, pc = i - h * pieces_head;
+      const u32x4 v = *(const u32x4 *)(q + (int64_t)token * q_stride_token +
+                                       (int64_t)(head_first + (int)h) * q_stride_head + 16 * pc);
+      *(u32x4 *)(staged + (int64_t)r * staged_row_stride + 16 * (int64_t)i) = v;
+    }
   }
 }
 
@@ -1864,9 +1867,11 @@ extern "C" int ekv_audit_stage_queries(const void *q, int q_dtype, int64_t q_str
   if (rows == 0) return EKV_OK;
   const int pieces = (int)(heads * (row_bytes / 16));
   const int threads = std::min(kStageThreads, (pieces + kWave - 1) / kWave * kWave);
-  hipLaunchKernelGGL(stage_queries_kernel, dim3((unsigned)rows, (unsigned)std::min((pieces + threads - 1) / threads, 65535)),
-                     dim3(threads), 0, (hipStream_t)stream, (const char *)q, q_stride_token * qbytes,
-                     q_stride_head * qbytes, head_first, heads, (int32_t)row_bytes, qrow, select, flag, (char *)staged,
-                     staged_row_stride * qbytes);
+  // a launch has fewer than 2^32 threads: past that a workgroup takes several rows
+  const dim3 grid(std::min((unsigned)rows, UINT_MAX / (unsigned)threads),
+                  (unsigned)std::min((pieces + threads - 1) / threads, 65535));
+  hipLaunchKernelGGL(stage_queries_kernel, grid, dim3(threads), 0, (hipStream_t)stream, (const char *)q,
+                     q_stride_token * qbytes, q_stride_head * qbytes, head_first, heads, (int32_t)row_bytes, qrow,
+                     select, flag, rows, (char *)staged, staged_row_stride * qbytes);
   return check_hip(hipGetLastError(), "ekv_audit_stage_queries launch");
 }

@@ -197,3 +197,27 @@ def test_captured_step_reads_the_queries_in_place():
         got = captured.read_planes()
         assert np.array_equal(got, want, equal_nan=True), f"replay {replay} differs from the eager staged step"
     assert (captured.read_cycles()[select] > 0).all()
+
+
+def test_staged_rows_past_the_thread_limit_of_a_launch():
+    # a workgroup of 64 threads a row would pass the 2^32 threads of a launch at 2^26 rows, so the
+    # workgroups take several; the selected rows are their queries exactly, the others untouched
+    if torch.cuda.mem_get_info()[0] < 4 << 30:
+        pytest.skip("needs 4 GiB of device memory")
+    import ekv_hip
+
+    rows, dim = (1 << 26) + 70, 8
+    q = torch.randn(9, 2, dim, device="cuda").to(torch.bfloat16)
+    chosen = torch.tensor([0, 63, 64, (1 << 26) - 2, (1 << 26) - 1, 1 << 26, rows - 1], device="cuda")
+    select = torch.zeros(rows, dtype=torch.uint8, device="cuda")
+    select[chosen] = 1
+    token = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    token[chosen] = torch.tensor([3, 8, 0, 5, 1, 7, 4], dtype=torch.int32, device="cuda")
+    staged = torch.zeros(rows, dim, dtype=torch.bfloat16, device="cuda")
+    for on in (0, 1):
+        flag = torch.tensor([on], dtype=torch.int32, device="cuda")
+        ekv_hip.call("ekv_audit_stage_queries", q.data_ptr(), ekv_hip.BF16, q.stride(0), q.stride(1), 1, 1, dim,
+                     token.data_ptr(), select.data_ptr(), flag.data_ptr(), rows, staged.data_ptr(), dim,
+                     ekv_hip.stream_handle())
+        assert torch.equal(staged[chosen], q[token[chosen].long(), 1] * on)
+        assert int(torch.count_nonzero(staged.any(dim=1))) == on * len(chosen)
