@@ -1375,23 +1375,30 @@ constexpr int reg_layers(int J) { return J == 1 ? 8 : (J == 4 ? 2 : 4); }
 
 // The stream form where its statistics fit the workspace (3 floats a cell and slice in each
 // (row, layer)'s width of partials) and it is the faster one, else false with nothing launched.
-// Against the partial-sum forms, over 250 shapes of 1-256 rows, 16-8192 blocks, 1-48 layers, it is up to
-// 10 times as fast where it is taken (0.94-1 at the lines drawn here) and its error against float64 no
-// larger (2.4-6.6e-8, 4.5-14e-8 before).  Where it is not taken: 4 cells and at most 1024 blocks from 64
-// rows or 769 blocks on, whose records the register form reads once (below that 1.1-1.26 times; 0.93 at
-// 16 x 1024, 0.68-0.86 at 128 and 256 rows, whose combines fill the GPU); 4096 and more short records of
-// several cells (0.91-0.94 at 200 rows x 32 layers x 128 blocks x 8 cells); single floats below 2048
-// floats and 512 blocks a record (0.62-1.14, 1.1-7 from there on); records of one cell below 64 blocks
-// (0.9 at 3 x 16), for the max below 512 (0.92 at 240 x 232).
+// Against the partial-sum forms, over 1000 shapes of 1-256 rows, 16-8192 blocks, 1-48 layers, it is up to
+// 10 times as fast where it is taken (1.6 to 2 in the mean) and its error against float64 no larger
+// (2.4-6.6e-8, 4.5-14e-8 before).  Where it is not taken (and its speed there against theirs): 4 cells and at
+// most 1024 blocks from 64 rows, 769 blocks or 700 records on, which the register form reads once (0.78-0.98
+// at 32 to 63 rows x 32 layers; 1.03 in the mean below); short records of several cells, from 1500 of them
+// on past 1024 floats (0.85-0.93) and from 4096 below; single floats below 512 blocks and 2048 floats a
+// record (0.62-1.14), 2560 past 9 cells (0.82-0.98), or from 128 rows of at most 5 layers on (0.83-0.93);
+// records of one cell below 64 blocks (0.9 at 3 x 16), for the max below 512 (0.92 at 240 x 232).  Taken and
+// lost: whole rows of single floats, many and of few layers (0.85 at 199 x 1933 x 1 layer x 6 cells, 0.89 at
+// 202 x 2110 x 2 x 7; rows of mixed lengths gain 1.2-1.6 there).
 bool launch_stream(Params p, int nrows, hipStream_t s) {
   if (p.from_u || nrows > kMaxArrivalRows || (int64_t)p.layers * p.cells > kMaxStreamStats) return false;
   const bool aligned = ((uintptr_t)p.m % 16) == 0 && ((uintptr_t)p.l % 16) == 0 && p.layer_stride % 4 == 0 &&
                        p.row_stride % 4 == 0;
   const bool quads = aligned && p.cells % 4 == 0;                        // four cells of a block
   const bool blocks = aligned && p.cells == 1 && p.width % 4 == 0;       // four blocks of one cell
-  if (quads && p.cells == 4 && p.width <= 4 * kSplitThreads && (nrows >= 64 || p.width > 3 * kSplitThreads)) return false;
-  if (quads && (int64_t)nrows * p.layers >= 4096 && p.width * p.cells <= 2048) return false;
-  if (!quads && !blocks && p.width < 512 && p.width * p.cells < 2048) return false;
+  if (quads && p.cells == 4 && p.width <= 4 * kSplitThreads &&
+      (nrows >= 64 || p.width > 3 * kSplitThreads || nrows * p.layers >= 700))
+    return false;
+  if (quads && p.width * p.cells <= 2048 && (int64_t)nrows * p.layers >= (p.width * p.cells <= 1024 ? 4096 : 1500))
+    return false;
+  if (!quads && !blocks && p.width < 512 &&
+      (p.width * p.cells < (p.cells > 9 ? 2560 : 2048) || (nrows >= 128 && p.layers <= 5)))
+    return false;
   if (blocks && p.width < (p.aggregate == EKV_AGG_MAX ? 512 : 64)) return false;
   p.nrows = nrows;
   p.period = quads ? p.cells / 4 : blocks ? 1 : p.cells;
@@ -1411,12 +1418,18 @@ bool launch_stream(Params p, int nrows, hipStream_t s) {
   p.slice_units = ((units + p.slices - 1) / p.slices + 4 * A * kUnits - 1) / (4 * A * kUnits) * (4 * A * kUnits);
   p.slices = (units + p.slice_units - 1) / p.slice_units;
   p.stats = reinterpret_cast<Stat *>(p.part);
-  // apply_kernel: layer groups of waves until the workgroups cover the GPU about four times
+  // apply_kernel's layer groups: fewer layers a wave, for more workgroups.  A workgroup takes about as long
+  // as a wave's layers and 12 more, the launch as its workgroups and 5 for 4 CUs.  Over 1680 shapes this
+  // is within 1.1% of the best of 1, 2, 4 and 8 groups (at most 1.21 times); splitting until there were four
+  // workgroups a CU came 7% from it, and to 1.93 times (69 rows x 519 blocks x 7 layers x 6 cells: 32 us in
+  // 1863 workgroups, 22 in 483).
   auto chunks_of = [&](int columns) { return (units + columns * A - 1) / (columns * A); };
+  auto time_of = [&](int g) {
+    return (double)(12 + (p.layers + g - 1) / g) * (1.25 * cu_count() + (double)nrows * chunks_of(kApplyWaves / g));
+  };
   int groups = 1;
-  while (groups < kApplyWaves && 2 * groups <= p.layers &&
-         (int64_t)nrows * chunks_of(kApplyWaves / groups) < 4 * (int64_t)cu_count())
-    groups <<= 1;
+  for (int g = 2; g <= kApplyWaves && g <= p.layers; g <<= 1)
+    if (time_of(g) < time_of(groups)) groups = g;
   p.columns = kApplyWaves / groups;
   p.chunks = chunks_of(p.columns);
   const int64_t grid1 = team ? records * p.slices : (records + 3) / 4, grid2 = (int64_t)nrows * p.chunks;
