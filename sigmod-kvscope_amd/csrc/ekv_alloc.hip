@@ -23,8 +23,8 @@
 // the lowest request first (observe/allocation.py:126-166).  Per request: the pinned shares' NumPy
 // sum (base), its open blocks in stable descending share order (by rank in buckets of the same
 // order-preserving keys, one workgroup per request, in LDS; a radix sort past 8192 blocks, in global
-// memory past 12288), and their running float64 totals, added in that order as np.cumsum does.  The 60-step bisection of the level: a request's count at a level is
-// min(1 + lower_bound(totals + 2 r, level - base - 1e-12 + 2 r), open), the shifted-by-2r comparison
+// memory past 12288), and their running float64 totals, added in that order as np.cumsum does.  The
+// 60-step bisection of the level: a request's count at a level is min(1 + lower_bound(totals + 2 r, level - base - 1e-12 + 2 r), open), the shifted-by-2r comparison
 // NumPy's single search makes.  Its first 20 steps are walks over counts that two kernels sum over
 // every CU at the levels they can reach; the rest run in one workgroup, every request keeping the
 // bracket of positions its count can still take.  The leftover goes to the requests tied at the
@@ -382,17 +382,17 @@ __device__ void pick_digit(const Params &p, int shift, int bits, int last_gain_p
 
 // One radix pass: the histogram of the `bits`-wide digit at `shift` over the open blocks whose key
 // matches the prefix so far (tie passes: the blocks at the gain threshold, over the tie key).
-// Workgroup w takes rows w, w + grid, ..., so each workgroup adds its LDS histogram into the global
-// one once, with device-scope atomics; once they have completed it counts its arrival, and the
-// pass's last workgroup picks the digit (pick_digit), so no second kernel runs per pass.
+// A workgroup takes its workers' rows (PassRows) and adds its LDS histogram into the global one once,
+// with device-scope atomics; once they have completed it counts its arrival, and the pass's last
+// workgroup picks the digit (pick_digit), so no second kernel runs per pass.
 // last_gain_pass: 1 on the last gain pass, 0 on the others, -1 on tie passes.
 // CAND_MODE: 1 (the second gain pass) also lists the blocks it counts, every one matching the first
 // pass's digit, in p.cand; 2 (the later passes) reads that list instead of the rows, unless it
 // outgrew its capacity.
 constexpr int kCandPerRow = 1024;  // the list's room per request row
-// The passes run one workgroup of kHistThreads per CU at most (rows w, w + grid, ... each): a pass's
-// workgroups each add their histogram into the global one, and the adds to one digit from every
-// workgroup are serialised in memory, so fewer, larger workgroups end the pass sooner.
+// The passes run one workgroup of kHistThreads per CU at most (its rows: PassRows): a pass's workgroups
+// each add their histogram into the global one, and the adds to one digit from every workgroup are
+// serialised in memory, so fewer, larger workgroups end the pass sooner.
 constexpr int kHistThreads = 1024;
 
 // A row of a pass is SPAN threads', so a workgroup takes kHistThreads / SPAN rows side by side: worker v
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(kHistThreads) void hist_kernel(const Params p, int 
       count(counted, digit);
     }
   } else {
-    // rows w, w + G, ... kHistRows at a time: every row's blocks of a step loaded before any is
+    // the worker's rows (each G after the last), kHistRows at a time: every row's blocks of a step loaded before any is
     // counted (a step's list stores then wait for no load of the same step).  The second pass also
     // writes the keep of every block the first digit decides (pinned and past-the-row blocks 1, an
     // open block 1 or 0 as its digit is above or below the threshold's), across the whole width, and
@@ -737,8 +737,8 @@ __device__ __forceinline__ void base_default(const MaxminParams &m, int r) {
 // A pass: each of the 16 waves owns a run of 64 * ITEMS consecutive positions and ranks it 64
 // positions (one per lane) at a time.  The lanes that share a digit are found from eight ballots of
 // its bits; a lane's rank in its wave is the wave's count of its digit so far (in LDS) plus the lanes
-// before it that share the digit, and those lanes store the count raised by their number.  The waves' counts, scanned digit by digit (descending) then wave by wave,
-// give each digit's first position for each wave, and every element moves to its place.  Equal digits
+// before it that share the digit, and those lanes store the count raised by their number.  The waves'
+// counts, scanned digit by digit (descending) then wave by wave, give each digit's first position for each wave, and every element moves to its place.  Equal digits
 // keep their order, so the passes compose into a stable sort.
 constexpr int kSortThreads = 1024;
 constexpr int kSortWaves = kSortThreads / kWave;
@@ -1498,8 +1498,8 @@ __global__ __launch_bounds__(kTotalsThreads) void mm_totals_kernel(const MaxminP
 // The sort places every open block by its exact rank, without passes over digits.  With x = (largest
 // key) - key, ascending in the sorted order, the blocks of positive shares are counted in 511 coarse bins
 // of x's leading bits (the zero shares follow in block order); a bin of c blocks is cut into about c / 2
-// to c / 4 buckets (two at least where the words below need it) of its next bits, so that a bucket holds a few blocks however the shares are spread;
-// and each block's rank is its bucket's first position plus the blocks of its bucket before it, counted
+// to c / 4 buckets (two at least where the words below need it) of its next bits, so that a bucket holds a
+// few blocks however the shares are spread; and each block's rank is its bucket's first position plus the blocks of its bucket before it, counted
 // by comparing.  A bucket's bits fix all but x's low 51 bits (shares over more than 2^9 binades take the
 // radix sort), so those and the block's 13-bit index are one 64-bit word, and every comparison is of the
 // whole key and then the index: the order is the stable one whatever order the buckets were filled in.

@@ -133,7 +133,6 @@ template <int NT, bool IN_LDS = false, class Get>
 __device__ double block_numpy_sum(Get get, int n, PairwiseLds &lds) {
   static_assert(NT % kWave == 0 && NT >= kPairNodes && NT <= 1024, "whole waves, a thread per tree node");
   constexpr int kPer = 16;  // values per accumulator in a leaf of at most 128
-  constexpr int H = NT >= 8 * 65 ? 1 : 2;  // chains a thread takes together (a run has at most 65 leaves)
   const int t = threadIdx.x, k = t & 7;
   const int v = t + 1;  // this thread's tree node (heap numbering), when v < kPairNodes
   const int depth = v < kPairNodes ? 31 - __clz(v) : 0;
@@ -186,51 +185,52 @@ __device__ double block_numpy_sum(Get get, int n, PairwiseLds &lds) {
           lds.node[lds.node_of[c >> 3]] = res;
         }
       }
-    } else
-    for (int c = t; c < chains; c += H * NT) {
-      double x[H][kPer], tail[H][7];
-      int m[H], rest[H];
+    } else {
+      for (int c = t; c < chains; c += 2 * NT) {
+        double x[2][kPer], tail[2][7];
+        int m[2], rest[2];
 #pragma unroll
-      for (int h = 0; h < H; ++h) {  // chains c and c + NT: every load issued before any add
-        const int cc = c + h * NT;
-        const int j = cc < chains ? cc >> 3 : 0;
-        const int s = lds.start[j], len = cc < chains ? lds.len[j] : 0;
-        m[h] = len >> 3;
-        rest[h] = len - 8 * m[h];
-        // every load issued, the unused ones reading value c0 (a load under a condition is followed
-        // by a wait for every load before it)
+        for (int h = 0; h < 2; ++h) {  // chains c and c + NT: every load issued before any add
+          const int cc = c + h * NT;
+          const int j = cc < chains ? cc >> 3 : 0;
+          const int s = lds.start[j], len = cc < chains ? lds.len[j] : 0;
+          m[h] = len >> 3;
+          rest[h] = len - 8 * m[h];
+          // every load issued, the unused ones reading value c0 (a load under a condition is followed
+          // by a wait for every load before it)
 #pragma unroll
-        for (int i = 0; i < kPer; ++i) {
-          const double y = get(i < m[h] ? s + k + 8 * i : c0);
-          x[h][i] = i < m[h] ? y : 0.0;
+          for (int i = 0; i < kPer; ++i) {
+            const double y = get(i < m[h] ? s + k + 8 * i : c0);
+            x[h][i] = i < m[h] ? y : 0.0;
+          }
+#pragma unroll
+          for (int i = 0; i < 7; ++i) {
+            const bool used = k == 0 && i < rest[h];
+            const double y = get(used ? s + 8 * m[h] + i : c0);
+            tail[h][i] = used ? y : 0.0;
+          }
         }
 #pragma unroll
-        for (int i = 0; i < 7; ++i) {
-          const bool used = k == 0 && i < rest[h];
-          const double y = get(used ? s + 8 * m[h] + i : c0);
-          tail[h][i] = used ? y : 0.0;
-        }
-      }
+        for (int h = 0; h < 2; ++h) {
+          const int cc = c + h * NT;
+          if (cc >= chains) continue;  // uniform over the eight threads of a leaf
+          double res = 0.0;
+          if (m[h] > 0) {
+            double r = x[h][0];
 #pragma unroll
-      for (int h = 0; h < H; ++h) {
-        const int cc = c + h * NT;
-        if (cc >= chains) continue;  // uniform over the eight threads of a leaf
-        double res = 0.0;
-        if (m[h] > 0) {
-          double r = x[h][0];
+            for (int i = 1; i < kPer; ++i)
+              if (i < m[h]) r += x[h][i];
+            r = r + __shfl_xor(r, 1, kWave);
+            r = r + __shfl_xor(r, 2, kWave);
+            r = r + __shfl_xor(r, 4, kWave);
+            res = r;
+          }
+          if (k == 0) {
 #pragma unroll
-          for (int i = 1; i < kPer; ++i)
-            if (i < m[h]) r += x[h][i];
-          r = r + __shfl_xor(r, 1, kWave);
-          r = r + __shfl_xor(r, 2, kWave);
-          r = r + __shfl_xor(r, 4, kWave);
-          res = r;
-        }
-        if (k == 0) {
-#pragma unroll
-          for (int i = 0; i < 7; ++i)
-            if (i < rest[h]) res += tail[h][i];
-          lds.node[lds.node_of[cc >> 3]] = res;
+            for (int i = 0; i < 7; ++i)
+              if (i < rest[h]) res += tail[h][i];
+            lds.node[lds.node_of[cc >> 3]] = res;
+          }
         }
       }
     }

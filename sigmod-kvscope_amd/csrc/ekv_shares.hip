@@ -1111,7 +1111,7 @@ __global__ __launch_bounds__(kStreamThreads) void stats_kernel(const Params p) {
 }
 
 // Each block's shares from the records and their peaks and totals: a workgroup takes `columns` columns
-// of A units of a row, 16 / columns waves a column, each over its layers (group g of LG:
+// of A units of a row, kApplyWaves / columns waves a column, each over its layers (group g of LG:
 // [g layers / LG, (g + 1) layers / LG)); the groups' sums (or maxes) meet in LDS and are added in group
 // order.  The first records are requested before the statistics are read.  The row's last workgroup to
 // arrive clears the row's statistics, writes the blocks past the row and, for the max, renormalises

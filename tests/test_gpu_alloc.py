@@ -317,8 +317,8 @@ def test_maxmin_running_totals_are_numpy_cumsums_bit_for_bit():
 @pytest.mark.parametrize("masked", [False, True])
 def test_maxmin_rows_of_one_workgroup(width, masked):
     # requests of at most 8192 blocks go from scores to running totals in one workgroup: ranks from
-    # buckets of the shares' leading bits, or a radix sort when a bucket is too full (equal shares,
-    # zeros) or the shares span more than 512 binades; totals in workgroup-wide windows.  Lengths at the
+    # buckets of the shares' leading bits, or a radix sort when too many unequal shares crowd in one or
+    # the shares span more than 512 binades; totals in workgroup-wide windows.  Lengths at the
     # edges of a thread's blocks, a wave and the row; the totals bit for bit np.cumsum's, the keep the
     # oracle's (NaN and inf rows: the totals only)
     rng = np.random.default_rng(900 + width + masked)
@@ -488,16 +488,16 @@ def test_maxmin_float64_scores_zero_rows_and_long_rows():
 
 @pytest.mark.parametrize("spread", [2.0 ** -40, 2.0 ** -30, 2.0 ** -26])
 def test_maxmin_shares_that_differ_only_in_low_bits(spread):
-    # the per-request sort orders the top 40 bits of each share's key first and sorts again on all 64
-    # bits only when two neighbours agree there but are out of order below: shares a few float64
-    # ulps apart (1 + k * spread, a handful of distinct values per row) take that second sort, next to
-    # rows whose shares differ high up
+    # shares a few float64 ulps apart (1 + k * spread, a handful of distinct values per row), next to rows
+    # whose shares differ high up: the row kernel's bins span the row's own shares, so each value has a
+    # bucket (the radix sort's second sort: test_maxmin_rows_past_8192_blocks_sorted_again and
+    # test_maxmin_equal_shares_keep_block_order)
     rng = np.random.default_rng(int(-np.log2(spread)))
     scores = []
     for n in (8192, 4096, 3000, 1024, 700, 64):
         s = 0.5 * (1.0 + rng.integers(0, 7, size=n) * spread)
         if n == 3000:
-            s = rng.random(n)  # no close neighbours: the first sort stands
+            s = rng.random(n)  # no close neighbours
         scores.append(s)
     pinned = [oa.default_pins(len(s)) for s in scores]
     total = sum(len(s) for s in scores)
@@ -509,9 +509,8 @@ def test_maxmin_shares_that_differ_only_in_low_bits(spread):
 
 
 def test_maxmin_ties_in_rows_sorted_in_lds():
-    # each request's blocks are sorted in LDS (a stable radix sort by share desc, so equal shares keep
-    # block order): rows full of exactly equal shares must keep the stable order the reference's
-    # argsort gives
+    # each request's blocks are ranked in LDS by share desc, equal shares in block order: rows full of
+    # exactly equal shares must keep the stable order the reference's argsort gives
     rng = np.random.default_rng(9)
     scores = [np.round(rng.random(n) * 8) / 8 for n in (8192, 4097, 1000, 64)]  # 9 distinct values
     scores.append(np.full(300, 0.25))
@@ -728,7 +727,7 @@ def test_maxmin_totals_with_many_ties_in_a_window(width, threads, masked):
 def test_maxmin_equal_shares_keep_block_order(width, masked):
     # more than 64 blocks in one of the ranks' buckets: of one share they are put in block order from a
     # bitmap; up to 128 of several shares are ranked by comparing, more send the request to the radix
-    # sort.  Group sizes around both limits, one group, as many groups as fit (short and whole rows), in
+    # sort and its second sort, on equal top bits (with each number of keys a thread).  Group sizes around both limits, one group, as many groups as fit (short and whole rows), in
     # random block order; the order read from the workspace
     rng = np.random.default_rng(width + masked)
     scores, pins = [], []
@@ -747,7 +746,7 @@ def test_maxmin_equal_shares_keep_block_order(width, masked):
             row(1.0 + np.arange(n) // size)
             row(np.where(np.arange(n) % 3, 2.0 ** -(1.0 + np.arange(n) // size % 40), 0.0))
     # one far share widens the bins, so that neighbouring float64 values share a bucket
-    for size in (60, 64, 65, 100, 128, 129, 200):
+    for size in (60, 64, 65, 100, 128, 129, 200, *sorted({min(n, width - 2) for n in (900, 1800, 3500, 8190)})):
         crowd = 1.0 + rng.integers(0, 3, size) * 2.0 ** -52
         row(np.concatenate([crowd, [1e-30, 1e-30], np.full(min(width - size - 2, 150), 2.0)]))
     row(np.concatenate([np.full(64, 1.0), [1.0 + 2.0 ** -52], [1e-30, 1e-30]]))
