@@ -22,7 +22,6 @@
 //    each lane's slice with the query slice (v_dot2 / FMA) and reduces over the lanes of a row.
 //  * Timer.  With a cycles buffer each wave adds its s_memtime durations to cycles[row] with a
 //    vector 64-bit atomic (the pass's per-row timer, mlir_pass/lib/eKVTimer.cpp:1348-1387).
-#include <limits.h>
 #include <math.h>
 
 #include <algorithm>
@@ -1276,8 +1275,8 @@ __global__ __launch_bounds__(kCuThreads) void tile_lse_layers_kernel(const Param
 
 // The step's queries staged per layer, for a launch that audits several layers after they have
 // run: staged[r][h][:] = q[qrow[r]][head_first + h][:] for the selected rows (nothing with the flag
-// off).  A workgroup copies (a part of) one row, a 16-byte piece a thread: every KV head's queries of 128
-// rows (1 MB) 5.1 us, which 8 workgroups of 16 rows had copied in 32 dependent turns each in 22.6 us.
+// off).  A workgroup copies (a part of) a row at a time, a 16-byte piece a thread: every KV head's queries of
+// 128 rows (1 MB) 5.1 us, which 8 workgroups of 16 rows had copied in 32 dependent turns each in 22.6 us.
 constexpr int kStageThreads = 256;  // at most; a row of fewer pieces takes as many waves as it has
 
 __global__ __launch_bounds__(kStageThreads) void stage_queries_kernel(
@@ -1867,9 +1866,10 @@ extern "C" int ekv_audit_stage_queries(const void *q, int q_dtype, int64_t q_str
   if (rows == 0) return EKV_OK;
   const int pieces = (int)(heads * (row_bytes / 16));
   const int threads = std::min(kStageThreads, (pieces + kWave - 1) / kWave * kWave);
-  // a launch has fewer than 2^32 threads: past that a workgroup takes several rows
-  const dim3 grid(std::min((unsigned)rows, UINT_MAX / (unsigned)threads),
-                  (unsigned)std::min((pieces + threads - 1) / threads, 65535));
+  // at most eight workgroups a CU of an MI355X, each with several rows past that: 8192 rows with the flag off 2.3
+  // us (3.5 a workgroup a row, 2.2 with 16 rows each), 8192 x 32 heads x 128 selected 21.6 (21.1, 32.9)
+  const unsigned parts = (unsigned)std::min((pieces + threads - 1) / threads, 65535);
+  const dim3 grid(std::min((unsigned)rows, std::max(1u, 2048u / parts)), parts);
   hipLaunchKernelGGL(stage_queries_kernel, grid, dim3(threads), 0, (hipStream_t)stream, (const char *)q,
                      q_stride_token * qbytes, q_stride_head * qbytes, head_first, heads, (int32_t)row_bytes, qrow,
                      select, flag, rows, (char *)staged, staged_row_stride * qbytes);

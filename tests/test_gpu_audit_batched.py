@@ -200,8 +200,8 @@ def test_captured_step_reads_the_queries_in_place():
 
 
 def test_staged_rows_past_the_thread_limit_of_a_launch():
-    # a workgroup of 64 threads a row would pass the 2^32 threads of a launch at 2^26 rows, so the
-    # workgroups take several; the selected rows are their queries exactly, the others untouched
+    # a workgroup of 64 threads a row would pass the 2^32 threads of a launch at 2^26 rows; at most 2048
+    # workgroups take several rows each; the selected rows are their queries exactly, the others untouched
     if torch.cuda.mem_get_info()[0] < 4 << 30:
         pytest.skip("needs 4 GiB of device memory")
     import ekv_hip
